@@ -467,124 +467,367 @@ __global__ void __launch_bounds__(256)
   teacher_slot(i, k, pos, vel, cs, bpos, bcs, g, u, radius, y, fine_pos, fine_vel);
 }
 
-// ---- training: generic bf16 GEMM (fp32 out) ---------------------------------
-// C[m][n] = sum_k A(m,k) B(k,n), A(m,k) = A[m sam + k sak],
-// B(k,n) = B[k sbk + n sbn]; one wave per 16x16 tile of C, 4 waves a block.
-// Bounds are checked per element (zero fill), so any M, N, K work.
-struct GemmArgs {
-  const uint16_t *A;
-  const uint16_t *B;
-  float *C;
-  int M, N, K;
-  long long sam, sak, sbk, sbn;
-  int ldc;
+// ---- training -----------------------------------------------------------------
+// One block of 8 waves takes chunks of 32 samples through the whole network
+// and back: activations and gradients stay in LDS, the weight gradients in
+// registers (24 tiles of 16 x 16 per wave over all layers), and only the
+// block's partial gradient goes to memory, where k_grad_reduce sums the
+// blocks in order.  What bounds it is the chain of layers (9 barriers a
+// chunk, each with an LDS round trip and at most 8 dependent MFMAs), not
+// memory or MFMA rate, so the layers share one launch: a gradient was 23
+// launches (a strided 2-byte GEMM per product, bias / ReLU / mask / loss /
+// column-sum passes between them) and is 2.  Measured: a gradient, an Adam
+// update and a forward over 512 samples 217 -> 31 us (kernels 15.6 + 3.9 +
+// 3.4 + 9.2; the rest is the host's launches), over 8,192 samples 1371 ->
+// 44 us (30 + 5 + 4 + 11).
+//
+// v_mfma_f32_16x16x32_bf16 with k = 8 q + e for element e of lane (c, q) in
+// both operands: an operand is 8 consecutive elements of one row, so every
+// product reads rows whose contraction index is contiguous.  A hidden layer
+// is stored twice in LDS for that, [sample][feature] (the next layer's
+// contraction) and [feature][sample] (the weight gradient's).  Wave w owns
+// features 16 w .. 16 w + 15 of every hidden layer.
+constexpr int kChunk = 32;           // samples per pass = one MFMA k-step of the weight gradient
+constexpr int kRowF = kHid + 8;      // [sample][feature] row, padded (16-byte rows, no bank pile-up)
+constexpr int kRowS = kChunk + 8;    // [feature][sample] row, padded the same way
+constexpr int kGradWaves = 8;
+constexpr int kPartial = 49152 + 416;  // floats of one block's partial gradient
+constexpr int kGradBlocks = 128;       // at most this many partial gradients
+
+// 8 bfloat16 / 4 floats from memory of any element alignment.
+typedef bf16x8 bf16x8_u __attribute__((aligned(2)));
+typedef bf16x4 bf16x4_u __attribute__((aligned(2)));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
+__device__ __forceinline__ bf16x8 ld8(const uint16_t *p) {
+  return *reinterpret_cast<const bf16x8_u *>(p);
+}
+
+// Element e: W[n0 + e][k] of a row-major matrix of K columns (a weight
+// fragment whose contraction runs over rows).
+__device__ __forceinline__ bf16x8 ld8_rows(const uint16_t *__restrict__ W, int K, int n0, int k) {
+  bf16x8 v;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = (short)W[(n0 + e) * K + k];
+  return v;
+}
+
+__device__ __forceinline__ bf16x4 to_bf16x4(const f32x4 &v) {
+  return bf16x4{(short)to_bf16(v[0]), (short)to_bf16(v[1]), (short)to_bf16(v[2]),
+                (short)to_bf16(v[3])};
+}
+
+// The tile's 4 features of one sample (lane (c, q)) into both LDS layouts
+// (bf null: only [feature][sample]).
+__device__ __forceinline__ void put_tile(uint16_t *bf, uint16_t *fb, int f0, int smp,
+                                         const bf16x4 &h) {
+  if (bf) *reinterpret_cast<bf16x4 *>(bf + smp * kRowF + f0) = h;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) fb[(f0 + e) * kRowS + smp] = (uint16_t)h[e];
+}
+
+// out[s] = sum over KS k-steps of a[ks] times the [sample][feature] rows of
+// sample tile s.
+template <int KS>
+__device__ __forceinline__ void rows_product(const bf16x8 (&a)[KS], const uint16_t *bf, int c,
+                                             int q, f32x4 (&out)[2]) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      z = mfma32(a[ks], *reinterpret_cast<const bf16x8 *>(bf + (16 * s + c) * kRowF + 32 * ks +
+                                                          8 * q),
+                 z);
+    out[s] = z;
+  }
+}
+
+// acc[t] += G^T H over the chunk's samples: feature rows n0.. of G against
+// the 16 T rows of H.
+template <int T>
+__device__ __forceinline__ void weight_product(const uint16_t *gs, const uint16_t *hs, int n0,
+                                               int c, int q, f32x4 (&acc)[T]) {
+  const bf16x8 a = *reinterpret_cast<const bf16x8 *>(gs + (n0 + c) * kRowS + 8 * q);
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    acc[t] = mfma32(a, *reinterpret_cast<const bf16x8 *>(hs + (16 * t + c) * kRowS + 8 * q),
+                    acc[t]);
+}
+
+struct GradArgs {
+  const uint16_t *__restrict__ w;
+  const float *__restrict__ bias;
+  const uint16_t *__restrict__ x;
+  const float *__restrict__ target;
+  int B;
+  float *dW, *db;    // the gradient itself when the launch has one block
+  float *part;       // kPartial floats per block otherwise
+  float *sq;         // per-sample squared error, or null
 };
 
-__global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs a) {
-  const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int lane = threadIdx.x & 63;
-  const int tiles_n = (a.N + 15) / 16;
-  const int tiles = ((a.M + 15) / 16) * tiles_n;
-  if (wave >= tiles) return;  // whole waves exit together
-  const int m0 = (wave / tiles_n) * 16, n0 = (wave % tiles_n) * 16;
+__global__ void __launch_bounds__(64 * kGradWaves) k_mlp_grad(GradArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[kIn * kRowS];        // x^T
+  __shared__ __attribute__((aligned(16))) uint16_t hs[3][kHid * kRowS];    // H_l^T
+  __shared__ __attribute__((aligned(16))) uint16_t gs[2][kHid * kRowS];    // G^T, alternating
+  __shared__ __attribute__((aligned(16))) uint16_t rows[2][kChunk * kRowF];  // H or G rows
+  __shared__ float db4[2][kOutPad];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int c = lane & 15, q = lane >> 4;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < a.K; k0 += 16) {
-    bf16x4 av, bv;
+  const int f0 = 16 * w + 4 * q;  // this lane's first feature in a hidden tile
+  const float scale = 2.0f / (float)(kOut * a.B);
+  // weight fragments of the way back (contraction over rows: 2-byte
+  // gathers), loaded once
+  bf16x8 t4[1], t3[4], t2[4];
+  t4[0] = ld8_rows(a.w + kWOff4, kHid, 8 * q, 16 * w + c);
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    t3[ks] = ld8_rows(a.w + kWOff3, kHid, 32 * ks + 8 * q, 16 * w + c);
+    t2[ks] = ld8_rows(a.w + kWOff2, kHid, 32 * ks + 8 * q, 16 * w + c);
+  }
+  f32x4 w1[6], w2[8], w3[8], w4[2];  // weight gradients: tiles of rows 16 w (w4: columns 16 w)
+  f32x4 b1 = {0.0f, 0.0f, 0.0f, 0.0f}, b2 = b1, b3 = b1, b4[2] = {b1, b1};
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    if (t < 6) w1[t] = b1;
+    w2[t] = w3[t] = b1;
+    if (t < 2) w4[t] = b1;
+  }
+  const int chunks = (a.B + kChunk - 1) / kChunk;
+  for (int ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
+    const int base = ch * kChunk;
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    f32x4 z[2];
+    unsigned int mask[3] = {0u, 0u, 0u};  // bit 4 s + e of layer l: Z > 0
+    // hidden layer l's tile from its product z: bias, ReLU, both layouts
+    auto activate = [&](int l, uint16_t *bf, uint16_t *fb) {
+      const f32x4 b = *reinterpret_cast<const f32x4_u *>(a.bias + kHid * l + f0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        f32x4 v = z[s] + b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (v[e] > 0.0f) mask[l] |= 1u << (4 * s + e);
+          v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+        }
+        put_tile(bf, fb, f0, 16 * s + c, to_bf16x4(v));
+      }
+    };
+    // layer 1 from x (rows past the batch: zeros)
+    {
+      bf16x8 wf[3], xf[2][3];
+#pragma unroll
+      for (int ks = 0; ks < 3; ++ks) {
+        wf[ks] = ld8(a.w + kWOff1 + (16 * w + c) * kIn + 32 * ks + 8 * q);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int smp = base + 16 * s + c;
+          xf[s][ks] = smp < a.B ? ld8(a.x + (size_t)smp * kIn + 32 * ks + 8 * q) : zero8;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        z[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < 3; ++ks) {
+          z[s] = mfma32(wf[ks], xf[s][ks], z[s]);
+          // wave 3 s + ks keeps this fragment's x^T
+          if (w == 3 * s + ks) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              xs[(32 * ks + 8 * q + e) * kRowS + 16 * s + c] = (uint16_t)xf[s][ks][e];
+          }
+        }
+      }
+      activate(0, rows[0], hs[0]);
+    }
+    {
+      bf16x8 wf[4];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        wf[ks] = ld8(a.w + kWOff2 + (16 * w + c) * kHid + 32 * ks + 8 * q);
+      __syncthreads();
+      rows_product<4>(wf, rows[0], c, q, z);
+      activate(1, rows[1], hs[1]);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        wf[ks] = ld8(a.w + kWOff3 + (16 * w + c) * kHid + 32 * ks + 8 * q);
+      __syncthreads();
+      rows_product<4>(wf, rows[1], c, q, z);
+      activate(2, rows[0], hs[2]);
+      __syncthreads();
+    }
+    // output layer and loss gradient: wave s < 2 takes sample tile s
+    if (w < 2) {
+      const int smp = base + 16 * w + c;
+      float s2 = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+          y = mfma32(ld8(a.w + kWOff4 + (16 * t + c) * kHid + 32 * ks + 8 * q),
+                     *reinterpret_cast<const bf16x8 *>(rows[0] + (16 * w + c) * kRowF + 32 * ks +
+                                                       8 * q),
+                     y);
+        f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (smp < a.B && 16 * t + 4 * q < kOut) {
+          const f32x4 e = (y + *reinterpret_cast<const f32x4_u *>(a.bias + kBOff4 + 16 * t +
+                                                                  4 * q)) -
+                          *reinterpret_cast<const f32x4_u *>(a.target + (size_t)smp * kOut +
+                                                             16 * t + 4 * q);
+          s2 += (e[0] * e[0] + e[1] * e[1]) + (e[2] * e[2] + e[3] * e[3]);
+          g = e * scale;
+        }
+        b4[t] += g;
+        put_tile(rows[1], gs[0], 16 * t + 4 * q, 16 * w + c, to_bf16x4(g));
+      }
+      s2 += __shfl_xor(s2, 16, 64);
+      s2 += __shfl_xor(s2, 32, 64);
+      if (a.sq && q == 0 && smp < a.B) a.sq[smp] = s2;
+    }
+    __syncthreads();
+    // layer l's gradient of the features this lane holds: masked, summed
+    // into the bias gradient, both layouts
+    auto backward = [&](int l, f32x4 &b, uint16_t *bf, uint16_t *fb) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        f32x4 g = z[s];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!((mask[l] >> (4 * s + e)) & 1u)) g[e] = 0.0f;
+        b += g;
+        put_tile(bf, fb, f0, 16 * s + c, to_bf16x4(g));
+      }
+    };
+    {
+      // dW4: both row tiles against column tile w
+      const bf16x8 hv = *reinterpret_cast<const bf16x8 *>(hs[2] + (16 * w + c) * kRowS + 8 * q);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        w4[t] = mfma32(*reinterpret_cast<const bf16x8 *>(gs[0] + (16 * t + c) * kRowS + 8 * q),
+                       hv, w4[t]);
+    }
+    rows_product<1>(t4, rows[1], c, q, z);
+    backward(2, b3, rows[0], gs[1]);
+    __syncthreads();
+    weight_product<8>(gs[1], hs[1], 16 * w, c, q, w3);
+    rows_product<4>(t3, rows[0], c, q, z);
+    backward(1, b2, rows[1], gs[0]);
+    __syncthreads();
+    weight_product<8>(gs[0], hs[0], 16 * w, c, q, w2);
+    rows_product<4>(t2, rows[1], c, q, z);
+    backward(0, b1, nullptr, gs[1]);
+    __syncthreads();
+    weight_product<6>(gs[1], xs, 16 * w, c, q, w1);
+    __syncthreads();  // the next chunk overwrites every buffer
+  }
+  // the block's gradient
+  float *dW = gridDim.x == 1 ? a.dW : a.part + (size_t)blockIdx.x * kPartial;
+  float *db = gridDim.x == 1 ? a.db : dW + 49152;
+  auto put_weights = [&](float *o, int K, int n0, int k, const f32x4 &v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[(n0 + 4 * q + e) * K + k + c] = v[e];
+  };
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    if (t < 6) put_weights(dW + kWOff1, kIn, 16 * w, 16 * t, w1[t]);
+    put_weights(dW + kWOff2, kHid, 16 * w, 16 * t, w2[t]);
+    put_weights(dW + kWOff3, kHid, 16 * w, 16 * t, w3[t]);
+    if (t < 2) put_weights(dW + kWOff4, kHid, 16 * t, 16 * w, w4[t]);
+  }
+  // bias gradients: the 16 samples of a tile are the 16 lanes of a quarter
+  auto over_samples = [&](f32x4 v) {
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], o, 64);
+    return v;
+  };
+  b1 = over_samples(b1);
+  b2 = over_samples(b2);
+  b3 = over_samples(b3);
+  if (c == 0) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int k = k0 + 4 * q + e;
-      const int m = m0 + c, nn = n0 + c;
-      av[e] = (m < a.M && k < a.K) ? (short)a.A[m * a.sam + k * a.sak] : (short)0;
-      bv[e] = (nn < a.N && k < a.K) ? (short)a.B[k * a.sbk + nn * a.sbn] : (short)0;
+      db[kBOff1 + f0 + e] = b1[e];
+      db[kBOff2 + f0 + e] = b2[e];
+      db[kBOff3 + f0 + e] = b3[e];
     }
-    acc = mfma16(av, bv, acc);
   }
+  if (w < 2) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int m = m0 + 4 * q + e, nn = n0 + c;
-    if (m < a.M && nn < a.N) a.C[(size_t)m * a.ldc + nn] = acc[e];
-  }
-}
-
-// Z = C + bias (fp32, kept for the backward mask); H = bf16(relu(Z)).
-// last: only Z (the network output y), N = 24 of the padded 32 columns.
-__global__ void k_bias_act(int B, int N, int ldc, const float *__restrict__ C,
-                           const float *__restrict__ bias, float *__restrict__ Z,
-                           uint16_t *__restrict__ H, int last) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)B * N) return;
-  const int b = (int)(t / N), nn = (int)(t % N);
-  const float z = C[(size_t)b * ldc + nn] + bias[nn];
-  Z[(size_t)b * N + nn] = z;
-  if (!last) H[(size_t)b * N + nn] = to_bf16(z > 0.0f ? z : 0.0f);
-}
-
-// g = 2 (y - t) / (24 B) on the 24 outputs, 0 on the 8 padding columns;
-// G = bf16(g); sq[b] = sum of the sample's squared errors.
-__global__ void k_loss_grad(int B, const float *__restrict__ y, const float *__restrict__ t,
-                            float *__restrict__ g, uint16_t *__restrict__ G,
-                            float *__restrict__ sq) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const float scale = 2.0f / (float)(kOut * B);
-  float s = 0.0f;
-  for (int nn = 0; nn < kOutPad; ++nn) {
-    float gv = 0.0f;
-    if (nn < kOut) {
-      const float e = y[(size_t)b * kOut + nn] - t[(size_t)b * kOut + nn];
-      s = s + e * e;
-      gv = e * scale;
+    for (int t = 0; t < 2; ++t) {
+      const f32x4 v = over_samples(b4[t]);
+      if (c == 0)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) db4[w][16 * t + 4 * q + e] = v[e];
     }
-    g[(size_t)b * kOutPad + nn] = gv;
-    G[(size_t)b * kOutPad + nn] = to_bf16(gv);
   }
-  if (sq) sq[b] = s;
-}
-
-// g_prev = D * [Z > 0]; G_prev = bf16(g_prev).
-__global__ void k_mask(long long count, const float *__restrict__ D, const float *__restrict__ Z,
-                       float *__restrict__ g, uint16_t *__restrict__ G) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  const float v = Z[t] > 0.0f ? D[t] : 0.0f;
-  g[t] = v;
-  G[t] = to_bf16(v);
-}
-
-// db[n] = sum over b of g[b][n]: one block per column; thread t sums
-// samples t, t + 256, ... in order, then a fixed tree in LDS (the same
-// order on every run).
-__global__ void __launch_bounds__(256) k_colsum(int B, int N, const float *__restrict__ g,
-                                                float *__restrict__ db) {
-  __shared__ float part[256];
-  const int nn = blockIdx.x;
-  float s = 0.0f;
-  for (int b = threadIdx.x; b < B; b += 256) s = s + g[(size_t)b * N + nn];
-  part[threadIdx.x] = s;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) part[threadIdx.x] = part[threadIdx.x] + part[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) db[nn] = part[0];
+  if (threadIdx.x < kOutPad) db[kBOff4 + threadIdx.x] = db4[0][threadIdx.x] + db4[1][threadIdx.x];
 }
 
-__global__ void k_adam(int count, float *__restrict__ w, float *__restrict__ m,
-                       float *__restrict__ v, const float *__restrict__ g,
-                       uint16_t *__restrict__ wb, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * (gi * gi);
+// dW, db = the sum of the blocks' partial gradients, in block order within
+// each of 4 interleaved groups of blocks, then the groups in order.  One
+// block per 64 columns of 4 floats.
+__global__ void __launch_bounds__(256)
+    k_grad_reduce(const float *__restrict__ part, int blocks, float *__restrict__ dW,
+                  float *__restrict__ db) {
+  __shared__ f32x4 sum[4][64];
+  const int col = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;
+  const f32x4 *p = reinterpret_cast<const f32x4 *>(part);
+  f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (col < kPartial / 4) {
+    int b = grp;
+    for (; b + 12 < blocks; b += 16) {
+      const f32x4 v0 = p[(size_t)b * (kPartial / 4) + col];
+      const f32x4 v1 = p[(size_t)(b + 4) * (kPartial / 4) + col];
+      const f32x4 v2 = p[(size_t)(b + 8) * (kPartial / 4) + col];
+      const f32x4 v3 = p[(size_t)(b + 12) * (kPartial / 4) + col];
+      s = (((s + v0) + v1) + v2) + v3;
+    }
+    for (; b < blocks; b += 4) s += p[(size_t)b * (kPartial / 4) + col];
+  }
+  sum[grp][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (grp == 0 && col < kPartial / 4) {
+    const int l = threadIdx.x;
+    const f32x4 v = ((sum[0][l] + sum[1][l]) + sum[2][l]) + sum[3][l];
+    float *o = 4 * col < 49152 ? dW + 4 * col : db + (4 * col - 49152);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = v[e];
+  }
+}
+
+// One Adam update of the weights (i < nw) and the biases behind them, with
+// the copies inference reads.
+struct AdamArgs {
+  float *w, *mw, *vw, *b, *mb, *vb;
+  const float *dW, *db;
+  uint16_t *wb;
+  float *bias;
+  int nw, nb;
+  float lr, b1, b2, eps, c1, c2;
+};
+
+__global__ void __launch_bounds__(256) k_adam(AdamArgs a) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.nw + a.nb) return;
+  const bool isw = t < a.nw;
+  const int i = isw ? t : t - a.nw;
+  float *w = isw ? a.w : a.b, *m = isw ? a.mw : a.mb, *v = isw ? a.vw : a.vb;
+  const float gi = (isw ? a.dW : a.db)[i];
+  const float mi = a.b1 * m[i] + (1.0f - a.b1) * gi;
+  const float vi = a.b2 * v[i] + (1.0f - a.b2) * (gi * gi);
   m[i] = mi;
   v[i] = vi;
-  const float mh = mi * c1, vh = vi * c2;
-  const float wi = w[i] - (lr * mh) / (sqrtf(vh) + eps);
+  const float mh = mi * a.c1, vh = vi * a.c2;
+  const float wi = w[i] - (a.lr * mh) / (sqrtf(vh) + a.eps);
   w[i] = wi;
-  if (wb) wb[i] = to_bf16(wi);
+  if (isw)
+    a.wb[i] = to_bf16(wi);
+  else
+    a.bias[i] = wi;
 }
 
 __global__ void k_to_bf16(long long count, const float *__restrict__ x, uint16_t *__restrict__ h) {
@@ -642,6 +885,21 @@ __device__ __forceinline__ void stage_layer(uint16_t *__restrict__ dst,
       hi = *reinterpret_cast<const uint2 *>(row + k + 16);
     }
     reinterpret_cast<uint4 *>(dst)[f] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+  }
+}
+
+// Weights (49,152 bfloat16) in fragment order and biases (416) into LDS, the
+// output layer's in out_row_source's order.
+__device__ __forceinline__ void stage_network(uint16_t *__restrict__ W, float *__restrict__ bias,
+                                              const uint16_t *__restrict__ wts,
+                                              const float *__restrict__ bias_g) {
+  stage_layer(W + kWOff1, wts + kWOff1, kHid, kIn / 32);
+  stage_layer(W + kWOff2, wts + kWOff2, kHid, kHid / 32);
+  stage_layer(W + kWOff3, wts + kWOff3, kHid, kHid / 32);
+  stage_layer<true>(W + kWOff4, wts + kWOff4, kOutPad, kHid / 32);
+  for (int i = threadIdx.x; i < 416; i += blockDim.x) {
+    const int so = i < kBOff4 ? i : out_row_source(i - kBOff4);
+    bias[i] = so < 0 ? 0.0f : (i < kBOff4 ? bias_g[i] : bias_g[kBOff4 + so]);
   }
 }
 
@@ -802,14 +1060,7 @@ __global__ void __launch_bounds__(64 * WAVES)
   Packed3 ps[TILES], vs[TILES];
   load_features<TILES>(n, feat4, grp, groups, c, q, cur);
   load_samples<TILES>(n, flags, pos, vel, grp, c, fl, ps, vs);
-  stage_layer(W + kWOff1, wts + kWOff1, kHid, kIn / 32);
-  stage_layer(W + kWOff2, wts + kWOff2, kHid, kHid / 32);
-  stage_layer(W + kWOff3, wts + kWOff3, kHid, kHid / 32);
-  stage_layer<true>(W + kWOff4, wts + kWOff4, kOutPad, kHid / 32);
-  for (int i = threadIdx.x; i < 416; i += blockDim.x) {
-    const int so = i < kBOff4 ? i : out_row_source(i - kBOff4);
-    bias[i] = so < 0 ? 0.0f : (i < kBOff4 ? bias_g[i] : bias_g[kBOff4 + so]);
-  }
+  stage_network(W, bias, wts, bias_g);
   // the template offsets radius * T of this lane's two slots q and 4 + q
   float rt[2][3];
 #pragma unroll
@@ -874,6 +1125,47 @@ __global__ void __launch_bounds__(64 * WAVES)
   }
 }
 
+// The network's outputs y (n x 24) of sample-major bfloat16 features x, with
+// the inference kernel's weight staging and register-resident layers: one
+// launch where the training forward was four GEMMs, four bias passes and a
+// copy.  One 16-sample tile per wave.
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+    k_mlp_forward(int n, const uint16_t *__restrict__ x, const uint16_t *__restrict__ wts,
+                  const float *__restrict__ bias_g, float *__restrict__ y_out) {
+  __shared__ __attribute__((aligned(16))) uint16_t W[49152];
+  __shared__ __attribute__((aligned(16))) float bias[416];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, q = lane >> 4;
+  const int groups = (n + 15) / 16;
+  stage_network(W, bias, wts, bias_g);
+  __syncthreads();
+  for (int grp = blockIdx.x * WAVES + wave; grp < groups; grp += gridDim.x * WAVES) {
+    const int smp = 16 * grp + c;
+    const uint16_t *row = x + (size_t)(smp < n ? smp : n - 1) * kIn;
+    bf16x8 in[1][4];
+    bf16x4 h[1][8];
+    f32x4 y[1][2];
+#pragma unroll
+    for (int ks = 0; ks < 3; ++ks)
+      in[0][ks] = cat8(*reinterpret_cast<const bf16x4_u *>(row + 32 * ks + 4 * q),
+                       *reinterpret_cast<const bf16x4_u *>(row + 32 * ks + 16 + 4 * q));
+    in[0][3] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    hidden_layer<1, 3>(W + kWOff1, bias + kBOff1, in, h, lane);
+    operands<1>(h, in);
+    hidden_layer<1, 4>(W + kWOff2, bias + kBOff2, in, h, lane);
+    operands<1>(h, in);
+    hidden_layer<1, 4>(W + kWOff3, bias + kBOff3, in, h, lane);
+    operands<1>(h, in);
+    output_layer<1>(W + kWOff4, bias + kBOff4, in, y, lane);
+    if (smp < n) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        st3(y_out, 8ll * smp + 4 * t + q, y[0][t][0], y[0][t][1], y[0][t][2]);
+    }
+  }
+}
+
 // Layout probe: D = A B for one 16x16x16 tile (A, B row-major bf16).
 __global__ void k_mfma_probe(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                              float *__restrict__ D) {
@@ -901,67 +1193,6 @@ MlpConst mlp_const(const gg_mlp_config *c) {
   m.guard_floor = c->guard_floor;
   m.guard_side = c->guard_side;
   return m;
-}
-
-int gemm(const uint16_t *A, long long sam, long long sak, const uint16_t *B, long long sbk,
-         long long sbn, float *C, int ldc, int M, int N, int K, hipStream_t st) {
-  if (M <= 0 || N <= 0) return GG_OK;
-  GemmArgs a{A, B, C, M, N, K, sam, sak, sbk, sbn, ldc};
-  const long long tiles = (long long)((M + 15) / 16) * ((N + 15) / 16);
-  k_gemm_bf16<<<nblocks(tiles, 4), 256, 0, st>>>(a);
-  GG_LAUNCH_CHECK();
-  return GG_OK;
-}
-
-// Scratch of the training path for batch B.
-struct TrainScratch {
-  float *C, *Z[4], *g0, *g1, *dwork;
-  uint16_t *H[4], *G;
-};
-
-size_t train_scratch_layout(int B, TrainScratch *t, char *base) {
-  size_t off = 0;
-  auto take = [&](size_t bytes) {
-    char *p = base ? base + off : nullptr;
-    off += (bytes + 255) & ~(size_t)255;
-    return p;
-  };
-  const size_t b = (size_t)(B > 0 ? B : 0);
-  TrainScratch s{};
-  s.C = reinterpret_cast<float *>(take(b * kHid * 4));
-  for (int l = 0; l < 4; ++l) s.Z[l] = reinterpret_cast<float *>(take(b * kHid * 4));
-  s.g0 = reinterpret_cast<float *>(take(b * kHid * 4));
-  s.g1 = reinterpret_cast<float *>(take(b * kHid * 4));
-  s.dwork = reinterpret_cast<float *>(take(b * kHid * 4));
-  for (int l = 0; l < 4; ++l) s.H[l] = reinterpret_cast<uint16_t *>(take(b * kHid * 2));
-  s.G = reinterpret_cast<uint16_t *>(take(b * kHid * 2));
-  if (t) *t = s;
-  return off;
-}
-
-constexpr int kDimIn[4] = {kIn, kHid, kHid, kHid};
-constexpr int kDimOut[4] = {kHid, kHid, kHid, kOutPad};
-constexpr int kWOffs[4] = {kWOff1, kWOff2, kWOff3, kWOff4};
-constexpr int kBOffs[4] = {kBOff1, kBOff2, kBOff3, kBOff4};
-
-// Training-path forward: Z_l, H_l kept in scratch; y = Z_4 (B x 24).
-int train_forward(const uint16_t *wb, const float *bias, const uint16_t *x, int B,
-                  TrainScratch &s, hipStream_t st) {
-  const uint16_t *h = x;
-  int K = kIn;
-  for (int l = 0; l < 4; ++l) {
-    const int N = kDimOut[l];
-    // C[b][n] = sum_k h[b][k] W_l[n][k]
-    GG_TRY(gemm(h, K, 1, wb + kWOffs[l], 1, K, s.C, kHid, B, N, K, st));
-    const int Nz = (l == 3) ? kOut : N;
-    k_bias_act<<<nblocks((long long)B * Nz, 256), 256, 0, st>>>(B, Nz, kHid, s.C,
-                                                               bias + kBOffs[l], s.Z[l], s.H[l],
-                                                               l == 3 ? 1 : 0);
-    GG_LAUNCH_CHECK();
-    h = s.H[l];
-    K = N;
-  }
-  return GG_OK;
 }
 
 }  // namespace gg
@@ -1040,20 +1271,38 @@ extern "C" int gg_mlp_fine_targets(const gg_particles *coarse, const gg_particle
   return GG_OK;
 }
 
+// Scratch the training entry points accept: 5,376 bytes per sample.  Blocks
+// beyond the first keep their partial gradients there, as many as fit, so
+// gg_mlp_train_scratch_bytes adds what a launch at full width needs.
+static size_t train_scratch_min(int batch) { return (size_t)batch * 5376; }
+
+// Blocks of a gradient over a batch: one per chunk of 32 samples up to
+// kGradBlocks (more would add partial gradients, 198 KB each, faster than
+// they shorten the chain of chunks per block).
+static int grad_blocks(int batch, size_t scratch_bytes) {
+  const long long chunks = ((long long)batch + kChunk - 1) / kChunk;
+  const long long fit = (long long)(scratch_bytes / (kPartial * sizeof(float)));
+  long long nb = chunks < kGradBlocks ? chunks : kGradBlocks;
+  if (nb > fit) nb = fit;
+  return nb < 1 ? 1 : (int)nb;
+}
+
 extern "C" size_t gg_mlp_train_scratch_bytes(int batch) {
   if (batch <= 0) return 0;
-  return train_scratch_layout(batch, nullptr, nullptr);
+  const size_t full = (size_t)grad_blocks(batch, ~size_t(0) >> 1) * kPartial * sizeof(float);
+  return full > train_scratch_min(batch) ? full : train_scratch_min(batch);
 }
 
 extern "C" int gg_mlp_forward(const gg_mlp_weights *w, const uint16_t *x, int B, float *y,
                               void *scratch, size_t scratch_bytes, hipStream_t stream) {
   if (!w || !w->w_bf16 || !w->bias || !x || !y || B <= 0 || !scratch) return GG_ERR_INVALID;
-  if (scratch_bytes < gg_mlp_train_scratch_bytes(B)) return GG_ERR_WORKSPACE;
-  TrainScratch s;
-  train_scratch_layout(B, &s, static_cast<char *>(scratch));
-  GG_TRY(train_forward(w->w_bf16, w->bias, x, B, s, stream));
-  return hip_status(hipMemcpyAsync(y, s.Z[3], sizeof(float) * (size_t)B * kOut,
-                                   hipMemcpyDeviceToDevice, stream));
+  if (scratch_bytes < train_scratch_min(B)) return GG_ERR_WORKSPACE;
+  constexpr int kWaves = 8;
+  const int blocks = nblocks(((long long)B + 15) / 16, kWaves);
+  k_mlp_forward<kWaves><<<blocks < 1024 ? blocks : 1024, 64 * kWaves, 0, stream>>>(
+      B, x, w->w_bf16, w->bias, y);
+  GG_LAUNCH_CHECK();
+  return GG_OK;
 }
 
 extern "C" int gg_mlp_grad(const gg_mlp_weights *w, const uint16_t *x, const float *target,
@@ -1061,30 +1310,18 @@ extern "C" int gg_mlp_grad(const gg_mlp_weights *w, const uint16_t *x, const flo
                            size_t scratch_bytes, hipStream_t stream) {
   if (!w || !w->w_bf16 || !w->bias || !x || !target || !dW || !db || B <= 0 || !scratch)
     return GG_ERR_INVALID;
-  if (scratch_bytes < gg_mlp_train_scratch_bytes(B)) return GG_ERR_WORKSPACE;
-  TrainScratch s;
-  train_scratch_layout(B, &s, static_cast<char *>(scratch));
-  GG_TRY(train_forward(w->w_bf16, w->bias, x, B, s, stream));
-  // output layer: g (B x 32), G = bf16(g)
-  k_loss_grad<<<nblocks(B, 256), 256, 0, stream>>>(B, s.Z[3], target, s.g0, s.G, sq_err);
+  if (scratch_bytes < train_scratch_min(B)) return GG_ERR_WORKSPACE;
+  // partial gradients are read as 16-byte vectors
+  char *at = static_cast<char *>(scratch);
+  const size_t skip = (16 - ((uintptr_t)at & 15)) & 15;
+  const int blocks = grad_blocks(B, scratch_bytes > skip ? scratch_bytes - skip : 0);
+  float *part = reinterpret_cast<float *>(at + skip);
+  k_mlp_grad<<<blocks, 64 * kGradWaves, 0, stream>>>(
+      GradArgs{w->w_bf16, w->bias, x, target, B, dW, db, part, sq_err});
   GG_LAUNCH_CHECK();
-  float *g = s.g0, *gp = s.g1;
-  for (int l = 3; l >= 0; --l) {
-    const int K = kDimIn[l], N = kDimOut[l];
-    const uint16_t *hin = (l == 0) ? x : s.H[l - 1];
-    // dW_l[n][k] = sum_b G[b][n] h[b][k]
-    GG_TRY(gemm(s.G, 1, N, hin, K, 1, dW + kWOffs[l], K, N, K, B, stream));
-    k_colsum<<<N, 256, 0, stream>>>(B, N, g, db + kBOffs[l]);
+  if (blocks > 1) {
+    k_grad_reduce<<<nblocks(kPartial / 4, 64), 256, 0, stream>>>(part, blocks, dW, db);
     GG_LAUNCH_CHECK();
-    if (l == 0) break;
-    // D[b][k] = sum_n G[b][n] W_l[n][k]; g_prev = D * [Z_{l-1} > 0]
-    GG_TRY(gemm(s.G, N, 1, w->w_bf16 + kWOffs[l], K, 1, s.dwork, K, B, K, N, stream));
-    k_mask<<<nblocks((long long)B * K, 256), 256, 0, stream>>>((long long)B * K, s.dwork,
-                                                               s.Z[l - 1], gp, s.G);
-    GG_LAUNCH_CHECK();
-    float *tmp = g;
-    g = gp;
-    gp = tmp;
   }
   return GG_OK;
 }
@@ -1096,16 +1333,12 @@ extern "C" int gg_mlp_adam(gg_mlp_weights *w, const float *dW, const float *db, 
     return GG_ERR_INVALID;
   const float c1 = (float)(1.0 / (1.0 - std::pow((double)beta1, step)));
   const float c2 = (float)(1.0 / (1.0 - std::pow((double)beta2, step)));
-  k_adam<<<nblocks(GG_MLP_WEIGHTS, 256), 256, 0, stream>>>(GG_MLP_WEIGHTS, w->w_master, w->m_w,
-                                                          w->v_w, dW, w->w_bf16, lr, beta1,
-                                                          beta2, eps, c1, c2);
+  const AdamArgs a{w->w_master, w->m_w,  w->v_w,         w->b_master,   w->m_b, w->v_b, dW, db,
+                   w->w_bf16,   w->bias, GG_MLP_WEIGHTS, GG_MLP_BIASES, lr,     beta1,  beta2,
+                   eps,         c1,      c2};
+  k_adam<<<nblocks(GG_MLP_WEIGHTS + GG_MLP_BIASES, 256), 256, 0, stream>>>(a);
   GG_LAUNCH_CHECK();
-  k_adam<<<nblocks(GG_MLP_BIASES, 256), 256, 0, stream>>>(GG_MLP_BIASES, w->b_master, w->m_b,
-                                                         w->v_b, db, nullptr, lr, beta1, beta2,
-                                                         eps, c1, c2);
-  GG_LAUNCH_CHECK();
-  return hip_status(hipMemcpyAsync(w->bias, w->b_master, sizeof(float) * GG_MLP_BIASES,
-                                   hipMemcpyDeviceToDevice, stream));
+  return GG_OK;
 }
 
 extern "C" int gg_mlp_sync_weights(gg_mlp_weights *w, hipStream_t stream) {
