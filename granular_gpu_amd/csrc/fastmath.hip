@@ -1,12 +1,15 @@
 // gg_fast_math_check: the short correctly rounded square root, reciprocal
-// and quotient of the contact kernels (sqrt_core, rcp_core, div_core in
+// and quotient of the contact kernels (sqrt_rsq, rcp_core, div_core in
 // gg_device.hpp) against the compiler's full IEEE sequences (sqrtf, '/'),
 // input by input on the device.
 //   mode 0: x = every float bit pattern first .. first+count-1 that lies in
-//           [2^-96, max float]: sqrt_core(x) vs sqrtf(x);
-//   mode 1: d = every pattern in [2^-48, 2^64): rcp_core(d) vs 1.0f / d;
+//           [2^-96, max float]: sqrt_rsq(x) vs sqrtf(x), and the reciprocal
+//           refined from its rsq (where it raises no tie) vs 1 / sqrtf(x);
+//   mode 1: d = every pattern in [2^-48, 2^64): rcp_core(d) vs 1.0f / d; and
+//           its mantissa over counts (over the whole mode every mantissa
+//           meets every count in [1, 2048]): div_by_count vs '/';
 //   mode 2: pattern k gives the numerator n = 2^e (1 + m) with e, m from k's
-//           bits spread over [2^-80, 2^40], and a SplitMix64 hash of k the
+//           bits spread over [2^-92, 2^40], and a SplitMix64 hash of k the
 //           denominator d over [2^-48, 2^40] (the domains the friction
 //           quotient uses): div_core(n, d) vs n / d.
 // Mismatches are added to *mismatches (device).
@@ -40,14 +43,25 @@ __global__ void __launch_bounds__(256) k_fast_math_check(int mode, uint64_t firs
     if (mode == 0) {
       const float x = __uint_as_float(bits);
       if (!(x >= kSqrtFastMin && x <= 3.40282347e+38f)) continue;
-      bad += __float_as_uint(sqrt_core(x)) != __float_as_uint(sqrtf(x));
+      const float d = sqrtf(x);
+      float y;
+      bad += __float_as_uint(sqrt_rsq(x, y)) != __float_as_uint(d);
+      bool tie = false;
+      const float r = rcp_refine(d, y, tie);
+      bad += !tie && __float_as_uint(r) != __float_as_uint(1.0f / d);
     } else if (mode == 1) {
       const float d = __uint_as_float(bits);
       if (!(d >= 0x1p-48f && d < 0x1p64f)) continue;
       bad += __float_as_uint(rcp_core(d)) != __float_as_uint(1.0f / d);
+      // 32 counts per exponent; the domain's 112 exponents cover all 2048
+      const float n = __uint_as_float((bits & 0x007fffffu) | ((uint32_t)(127 - 30 + (bits >> 28)) << 23));
+      for (int t = 0; t < 32; ++t) {
+        const float kf = (float)(1 + (((bits >> 23) * 32 + t) & 2047));
+        bad += __float_as_uint(div_by_count(n, kf, rcp_core(kf))) != __float_as_uint(n / kf);
+      }
     } else {
       const uint64_t h = mix64(first + k);
-      const float n = in_range((uint64_t)bits * 0x9E3779B1ull, 127 - 80, 127 + 40);
+      const float n = in_range((uint64_t)bits * 0x9E3779B1ull, 127 - 92, 127 + 40);
       const float d = in_range(h, 127 - 48, 127 + 40);
       bad += __float_as_uint(div_core(n, d)) != __float_as_uint(n / d);
     }

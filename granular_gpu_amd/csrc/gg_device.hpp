@@ -12,18 +12,40 @@
 namespace gg {
 
 struct DevGrid {
-  float L;
+  float L, invL;  // cell length and the rounded 1 / L
   int cx, cy, cz;
 };
 
-inline DevGrid dev_grid(const gg_grid &g) { return DevGrid{g.cell_length, g.cx, g.cy, g.cz}; }
+inline DevGrid dev_grid(const gg_grid &g) {
+  return DevGrid{g.cell_length, 1.0f / g.cell_length, g.cx, g.cy, g.cz};
+}
+
+// q with the floor and truncation of the rounded quotients p / L: p (1/L) is
+// within 2^-22 |q| of them, so unless it is that close to a whole number
+// both lie on one side of every whole number.  (Three divisions are 33
+// instructions, this is 15; a wave meets a near-whole quotient about once in
+// 200, and then divides.)
+__device__ __forceinline__ void cell_quotient(float px, float py, float pz, const DevGrid &g,
+                                              float &qx, float &qy, float &qz) {
+  qx = px * g.invL;
+  qy = py * g.invL;
+  qz = pz * g.invL;
+  auto near_whole = [](float q) {
+    return !(fabsf(q - rintf(q)) > fabsf(q) * 0x1p-20f + 0x1p-100f);
+  };
+  if (near_whole(qx) || near_whole(qy) || near_whole(qz)) {
+    qx = px / g.L;
+    qy = py / g.L;
+    qz = pz / g.L;
+  }
+}
 
 // Cell id of a position: floor(p/L) per axis, x-major, sentinel C outside
 // the grid (CUDAFunctions.cuh:71-107).  NaN / huge coordinates -> sentinel.
 __device__ __forceinline__ int hash_cell(float px, float py, float pz, const DevGrid &g) {
-  const float fx = floorf(px / g.L);
-  const float fy = floorf(py / g.L);
-  const float fz = floorf(pz / g.L);
+  float qx, qy, qz;
+  cell_quotient(px, py, pz, g, qx, qy, qz);
+  const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
   if (!(fx >= 0.0f && fx < (float)g.cx && fy >= 0.0f && fy < (float)g.cy && fz >= 0.0f &&
         fz < (float)g.cz))
     return g.cx * g.cy * g.cz;
@@ -34,7 +56,8 @@ __device__ __forceinline__ int hash_cell(float px, float py, float pz, const Dev
 // (helper_math.h:176-179 as used in Solver.cu:382).
 __device__ __forceinline__ bool trunc_cell(float px, float py, float pz, const DevGrid &g, int &bx,
                                            int &by, int &bz) {
-  const float qx = px / g.L, qy = py / g.L, qz = pz / g.L;
+  float qx, qy, qz;
+  cell_quotient(px, py, pz, g, qx, qy, qz);
   const float lim = 1073741824.0f;
   if (!(qx > -lim && qx < lim && qy > -lim && qy < lim && qz > -lim && qz < lim)) return false;
   bx = (int)qx;
@@ -46,7 +69,11 @@ __device__ __forceinline__ bool trunc_cell(float px, float py, float pz, const D
 // Upsampler base: floorf(p / L) (Solver.cu:1271).
 __device__ __forceinline__ bool floor_cell(float px, float py, float pz, const DevGrid &g, int &bx,
                                            int &by, int &bz) {
-  const float qx = floorf(px / g.L), qy = floorf(py / g.L), qz = floorf(pz / g.L);
+  float qx, qy, qz;
+  cell_quotient(px, py, pz, g, qx, qy, qz);
+  qx = floorf(qx);
+  qy = floorf(qy);
+  qz = floorf(qz);
   const float lim = 1073741824.0f;
   if (!(qx > -lim && qx < lim && qy > -lim && qy < lim && qz > -lim && qz < lim)) return false;
   bx = (int)qx;
@@ -126,6 +153,7 @@ struct SweepConst {
   float rmin;      // clamp of r_i against the boundary
   float mu_s, mu_k;
   float half_valid;  // list usable while every displacement < half_valid
+  float near_valid;  // near list usable while the two displacements add up to less
   int gmax, bmax, cap;
 };
 
@@ -148,60 +176,70 @@ __device__ __forceinline__ LocalGrid local_grid(const SceneView &sv, int i, cons
   if (!SCENES) return LocalGrid{g0, 0, sc.mu_s, sc.mu_k};
   const int k = sv.scene_of[i];
   const gg_scene_desc d = sv.desc[k < 0 ? 0 : (k < sv.count ? k : sv.count - 1)];
-  return LocalGrid{DevGrid{g0.L, d.cx, d.cy, d.cz}, d.cell_base, d.mu_s, d.mu_k};
+  return LocalGrid{DevGrid{g0.L, g0.invL, d.cx, d.cy, d.cz}, d.cell_base, d.mu_s, d.mu_k};
 }
 
 // Correctly rounded square root, reciprocal and quotient on restricted
-// domains.  The compiler's IEEE sequences (what sqrtf and '/' compile to
-// under -fhip-fp32-correctly-rounded-divide-sqrt) wrap a core in steps that
-// are identities on these domains: for sqrt, the input scaling below 2^-96
-// and the +-0 / +inf class check; for division, v_div_scale (no scaling when
-// numerator and denominator are normal, the numerator's biased exponent
-// exceeds 23, the exponent difference is below 96 and neither 1/d nor n/d
-// is denormal), v_div_fmas (a plain fma when not scaled) and v_div_fixup
-// (pass-through for finite normal quotients).  The cores below are those
-// sequences without the identity steps, so their results equal sqrtf and
-// '/' bit for bit on the domains (checked over every input by
-// gg_fast_math_check); callers fall back to sqrtf and '/' outside them.
-constexpr float kSqrtFastMin = 0x1p-96f;  // sqrt_core domain [2^-96, max float]
+// domains, shorter than the compiler's IEEE sequences (what sqrtf and '/'
+// compile to under -fhip-fp32-correctly-rounded-divide-sqrt).  Those wrap a
+// core in scaling, pass-through and fixup steps that are identities on the
+// domains, and start the square root and the reciprocal from an
+// approximation each (v_sqrt_f32, v_rcp_f32: quarter-rate instructions).
+// Here the root is one Newton step with an exact residual from x rsq(x), and
+// in the list path the same v_rsq_f32 starts the reciprocal.  The results
+// equal sqrtf and '/' bit for bit: gg_fast_math_check compares them over
+// every float of the domains; callers fall back to sqrtf and '/' outside
+// them.  Per contact with friction (two roots, a reciprocal and a quotient)
+// this is 19 instructions, 2 of them quarter-rate, where the sequences
+// without the identity steps were 33 with 4.
+constexpr float kSqrtFastMin = 0x1p-96f;  // domain of the root: [2^-96, max float]
+
+// rsq and the root: d = sqrt(x), y = 1/sqrt(x) within an ulp.
+__device__ __forceinline__ float sqrt_rsq(float x, float &y) {
+  y = __builtin_amdgcn_rsqf(x);
+  const float s = x * y, h = 0.5f * y;
+  return __builtin_fmaf(__builtin_fmaf(-s, s, x), h, s);
+}
 
 __device__ __forceinline__ float sqrt_core(float x) {
-  float s = __builtin_amdgcn_sqrtf(x);
-  const float sm = __int_as_float(__float_as_int(s) - 1);
-  const float sp = __int_as_float(__float_as_int(s) + 1);
-  const float rm = __builtin_fmaf(-sm, s, x);
-  const float rp = __builtin_fmaf(-sp, s, x);
-  s = rm <= 0.0f ? sm : s;
-  s = rp > 0.0f ? sp : s;
-  return s;
+  float y;
+  return sqrt_rsq(x, y);
 }
 
-// n / d for normal n, d with the conditions above.
-__device__ __forceinline__ float div_core(float n, float d) {
-  const float r0 = __builtin_amdgcn_rcpf(d);
-  const float e0 = __builtin_fmaf(-d, r0, 1.0f);
-  const float r1 = __builtin_fmaf(e0, r0, r0);
-  const float q0 = n * r1;
-  const float e1 = __builtin_fmaf(-d, q0, n);
-  const float q1 = __builtin_fmaf(e1, r1, q0);
-  const float e2 = __builtin_fmaf(-d, q1, n);
-  return __builtin_fmaf(e2, r1, q1);
+// 1 / d from d = sqrt(x) and y = rsq(x), except where the step's residual
+// 1 - d y is 2^-24 (of all mantissas only d's all ones, where y (1 + 2^-24)
+// is a tie that rounds the wrong way): tie is raised there.
+__device__ __forceinline__ float rcp_refine(float d, float y, bool &tie) {
+  const float e = __builtin_fmaf(-d, y, 1.0f);
+  tie |= e == 0x1p-24f;
+  return __builtin_fmaf(e, y, y);
 }
 
-// 1 / d (the numerator is exactly 1, so n * r1 = r1).
+// 1 / d for d in [2^-48, 2^64) (no tie is left from v_rcp_f32).
 __device__ __forceinline__ float rcp_core(float d) {
-  const float r0 = __builtin_amdgcn_rcpf(d);
-  const float e0 = __builtin_fmaf(-d, r0, 1.0f);
-  const float r1 = __builtin_fmaf(e0, r0, r0);
-  const float e1 = __builtin_fmaf(-d, r1, 1.0f);
-  const float q1 = __builtin_fmaf(e1, r1, r1);
-  const float e2 = __builtin_fmaf(-d, q1, 1.0f);
-  return __builtin_fmaf(e2, r1, q1);
+  const float y = __builtin_amdgcn_rcpf(d);
+  return __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
 }
 
-// d = sqrt(d2) and inv = 1/d, as sqrtf and 1.0f/d give them.  For d2 in
-// [2^-96, max float], d lies in [2^-48, 2^64), where 1/d meets the
-// division conditions.
+// n / d from r = the rounded 1 / d, for normal n and d (or n = 0) whose
+// quotient and remainders stay normal: n in [2^-92, 2^40], d in [2^-48, 2^40].
+__device__ __forceinline__ float div_by(float n, float d, float r) {
+  const float q0 = n * r;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-d, q0, n), r, q0);
+  return __builtin_fmaf(__builtin_fmaf(-d, q1, n), r, q1);
+}
+
+__device__ __forceinline__ float div_core(float n, float d) { return div_by(n, d, rcp_core(d)); }
+
+// n / k for a whole number k in [1, 2048] with r = the rounded 1 / k, and n
+// = 0 or |n| in [2^-80, 2^60]: one correction is enough there (checked for
+// every mantissa and k).
+__device__ __forceinline__ float div_by_count(float n, float k, float r) {
+  const float q = n * r;
+  return __builtin_fmaf(__builtin_fmaf(-k, q, n), r, q);
+}
+
+// d = sqrt(d2) and inv = 1/d, as sqrtf and 1.0f/d give them.
 __device__ __forceinline__ void sqrt_rcp(float d2, float &d, float &inv) {
   if (d2 >= kSqrtFastMin && d2 <= 3.40282347e+38f) {
     d = sqrt_core(d2);
@@ -216,8 +254,8 @@ __device__ __forceinline__ void sqrt_rcp(float d2, float &d, float &inv) {
 // inv = 1/d of the contact.  Static when |t|^2 < (mu_s delta)^2 (squares:
 // the static case needs no square root); otherwise t scaled by
 // min(mu_k delta / |t|, 1).  In the kinetic case |t| = sqrt(tl2) with tl2
-// in [2^-96, 2^80] and mu_k delta in [2^-80, 2^40] keep the quotient inside
-// the division domain (quotient in [2^-120, 2^88]).
+// in [2^-96, 2^40] and mu_k delta in [2^-92, 2^40] keep the quotient inside
+// the division domain (quotient in [2^-112, 2^88]).
 __device__ __forceinline__ float3 friction(float px, float py, float pz, float inv, float delta,
                                            float rx, float ry, float rz, float mu_s, float mu_k) {
   const float nx = px * inv, ny = py * inv, nz = pz * inv;
@@ -230,10 +268,11 @@ __device__ __forceinline__ float3 friction(float px, float py, float pz, float i
   if (tl2 < lim * lim) return make_float3(tx, ty, tz);
   const float num = mu_k * delta;
   float c;
-  if (tl2 >= kSqrtFastMin && tl2 <= 0x1p80f && num >= 0x1p-80f && num <= 0x1p40f)
+  if (tl2 >= kSqrtFastMin && tl2 <= 0x1p40f && num >= 0x1p-92f && num <= 0x1p40f) {
     c = div_core(num, sqrt_core(tl2));
-  else
+  } else {
     c = num / sqrtf(tl2);
+  }
   c = fminf(c, 1.0f);
   return make_float3(tx * c, ty * c, tz * c);
 }
@@ -286,6 +325,73 @@ __device__ __forceinline__ bool granular_terms(const float4 &bi, const float4 &o
     f = friction(px, py, pz, inv, rc - d, rx, ry, rz, sc.mu_s, sc.mu_k);
   }
   return true;
+}
+
+// The same terms without branches for the list path of a sweep, where the
+// instruction count is the time: every lane evaluates every slot, lanes out
+// of contact add nothing.  Exact wherever it does not raise `redo`: a lane
+// that meets operands outside the short sequences' domains (positions less
+// than 2^-48 apart but distinct, tangential displacements below 2^-48 or
+// above 2^20, rcp_refine's tie: one contact in 10^7) is evaluated again with
+// the full sequences.  Callers
+// keep list_fast's conditions (radii below 2^60, so a contact's d2 is finite;
+// mu_k 0 or in [2^-20, 2^20], so that mu_k delta is 0 or in [2^-92, 2^40]
+// since delta = rc - d is 0 or at least an ulp of d).  d2 = 0 (coincident
+// particles, and the particle itself in a padding slot) gives d = NaN, which
+// is no contact, as d > 0 demands.
+constexpr unsigned int kSqrtFastMinBits = 0x0f800000u;  // 2^-96
+template <bool FRIC, bool STRICT>
+__device__ __forceinline__ bool fast_terms(float px, float py, float pz, float rx, float ry,
+                                           float rz, float rc, float mu_s, float mu_k, float3 &a,
+                                           bool &redo) {
+  const float d2 = px * px + py * py + pz * pz;
+  float y;
+  const float d = sqrt_rsq(d2, y);
+  redo |= __float_as_uint(d2) - 1u < kSqrtFastMinBits - 1u;
+  const bool hit = STRICT ? d < rc : d <= rc;
+  if (!hit) return false;
+  const float inv = rcp_refine(d, y, redo);
+  const float delta = rc - d;
+  const float s = delta * inv;
+  a.x = a.x + s * px;
+  a.y = a.y + s * py;
+  a.z = a.z + s * pz;
+  if (FRIC) {
+    const float nx = px * inv, ny = py * inv, nz = pz * inv;
+    const float rn = rx * nx + ry * ny + rz * nz;
+    const float tx = rx - rn * nx, ty = ry - rn * ny, tz = rz - rn * nz;
+    const float tl2 = tx * tx + ty * ty + tz * tz;
+    const float lim = mu_s * delta;
+    // t = 0 keeps t whatever the limit (min(NaN or inf, 1) = 1)
+    const bool fixed = tl2 < fmaxf(lim * lim, 1.401298464e-45f);
+    float yt;
+    const float dt = sqrt_rsq(tl2, yt);
+    const float c = fminf(div_by(mu_k * delta, dt, rcp_refine(dt, yt, redo)), 1.0f);
+    redo |= !fixed && __float_as_uint(tl2) - kSqrtFastMinBits > 0x53800000u - kSqrtFastMinBits;
+    const float f = fixed ? 1.0f : c;
+    a.x = a.x - tx * f;
+    a.y = a.y - ty * f;
+    a.z = a.z - tz * f;
+  }
+  return true;
+}
+
+// a / nf per component (nf >= 1 a whole number), as '/' gives it.
+__device__ __forceinline__ float3 mean_of(float ax, float ay, float az, float nf) {
+  const unsigned int ux = __float_as_uint(ax) & 0x7fffffffu, uy = __float_as_uint(ay) & 0x7fffffffu,
+                     uz = __float_as_uint(az) & 0x7fffffffu;
+  // 0 < |a| < 2^-80, or above 2^60 (NaN with it)
+  const bool odd = ux - 1u < 0x17800000u - 1u || uy - 1u < 0x17800000u - 1u ||
+                   uz - 1u < 0x17800000u - 1u || max(max(ux, uy), uz) > 0x5d800000u || nf > 2048.0f;
+  if (odd) return make_float3(ax / nf, ay / nf, az / nf);
+  const float r = rcp_core(nf);
+  return make_float3(div_by_count(ax, nf, r), div_by_count(ay, nf, r), div_by_count(az, nf, r));
+}
+
+// sqrtf(x) for x >= 0 (or NaN), the short sequence where it holds.
+__device__ __forceinline__ float sqrt_any(float x) {
+  if (__float_as_uint(x) - 1u < kSqrtFastMinBits - 1u || !(x <= 3.40282347e+38f)) return sqrtf(x);
+  return x == 0.0f ? 0.0f : sqrt_core(x);
 }
 
 // Adds one contact's terms: a + c, then - f (the order every path uses).

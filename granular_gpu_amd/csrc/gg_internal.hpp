@@ -23,6 +23,17 @@ constexpr float kPiF = 3.14159265358979323846f;
 // that of every particle of its stencil stay below half of this fraction of
 // the skin.
 constexpr float kListValidFrac = 0.9f;
+// Near lists: of a list's entries those within kNearFrac of the skin, at
+// most kNearMax of them.  They hold every contact while the displacements of
+// a pair add up to less than kNearValidFrac of the skin (the same 0.1 skin of
+// margin as above); unmarked neighbours have moved less than 0.45 skin, so a
+// particle reads its near list until it has moved 0.15 skin itself (1.1 mm of
+// the default 7.5, five times what one moves per step in a settled pile), and
+// its full list after that.  In a lattice this drops the second shell: a
+// third of the gathers, which is what a sweep's time follows.
+constexpr float kNearFrac = 0.7f;
+constexpr float kNearValidFrac = 0.6f;
+constexpr int kNearMax = 15;
 // A wave with at most this many particles that must scan the full stencil
 // queues them for one wave each (else each scans in its own lane), in its
 // block's LDS queue, scanned by the block's waves after their list work.
@@ -74,6 +85,8 @@ struct Layout {
   size_t v3tmp1;   // float3[cmax]
   size_t bnd4;     // float4[bcap]   packed sorted boundary
   // adaptive merge/split
+  size_t near;     // int[(kNearMax + 1) * cap]  near lists, over the arrays from cover to
+                   //                mrad (64 bytes a particle), within one step only
   size_t cover;    // float4[cap]    cover vectors
   size_t cand;     // int[cap]       merge candidate
   size_t dens;     // float[cap]     local density
@@ -141,6 +154,8 @@ inline Layout make_layout(int capacity, int bcap, gg_grid g, int max_sweeps,
   L.v3tmp1 = take(cmax * 12);
   L.bnd4 = take(((size_t)bcap + 1) * 16);
   const size_t nblk = (cap + kBlock - 1) / kBlock + 2;
+  L.near = o;
+  static_assert((kNearMax + 1) * 4 <= 16 + 7 * 4 + 16 + 4, "near lists fit the adaptive arrays");
   L.cover = take(cap * 16);
   L.cand = take(cap * 4);
   L.dens = take(cap * 4);

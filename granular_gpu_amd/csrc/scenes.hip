@@ -30,7 +30,7 @@ __global__ void __launch_bounds__(kBlock)
   k = k < 0 ? 0 : (k < count ? k : count - 1);
   const gg_scene_desc d = desc[k];
   const Packed3 p = ld3(pos, i);
-  keys[i] = d.cell_base + hash_cell(p.x, p.y, p.z, DevGrid{L, d.cx, d.cy, d.cz});
+  keys[i] = d.cell_base + hash_cell(p.x, p.y, p.z, DevGrid{L, 1.0f / L, d.cx, d.cy, d.cz});
 }
 
 int check_scenes(const gg_scenes *sc, const gg_workspace *ws) {
