@@ -13,9 +13,9 @@ namespace gg {
 constexpr int kBlock = 256;        // threads per block for particle kernels
 constexpr int kScanTile = 2048;    // elements per block in the cell-table scan
 constexpr int kScanMaxParts = 8192;
-constexpr int kSmallCell = 32;     // cells up to this size are ranked one thread per entry
-constexpr int kBigLds = 4096;      // cells up to this size are sorted in LDS
+constexpr int kBigLds = 4096;      // cells up to this size are ranked one thread per entry
 constexpr int kHugeChunks = 256;   // blocks compacting each larger cell
+constexpr int kScanSync = 8;       // ctr2[8..9]: the scan's tile and finish counters
 constexpr int kHugeCounter = 63;   // ctr[63]: cells larger than kBigLds in this build
 constexpr double kPiD = 3.14159265358979323846;
 constexpr float kPiF = 3.14159265358979323846f;
@@ -60,10 +60,10 @@ struct Layout {
   size_t slot;     // int[cmax]      arrival slot inside the cell
   size_t perm;     // int[cmax]      sorted slot -> old index
   size_t itmp;     // int[cmax]      cell order as scattered (before the stable ranking)
-  size_t part;     // int[parts+1]   scan partials
-  size_t big;      // int[C+1]       list of cells needing the big sort
-  size_t ctr;      // int[64]        device counters ([0] = big-cell count)
-  size_t ctr2;     // int[64]        adaptive counters
+  size_t part;     // int[parts+1]   scan tile states, zero between scans
+  size_t big;      // int[C+1]       record of each cell of more than kBigLds members
+  size_t ctr;      // int[64]        device counters
+  size_t ctr2;     // int[64]        adaptive and scan counters
   size_t dirty;    // int[C+1]       cells near a particle past half the skin
   size_t bounds;   // uint[4]        largest |D| component and contact radius of the step (float bits)
   size_t bpart;    // uint[2*blocks] per-block maxima reduced into bounds

@@ -5,9 +5,10 @@
 // CUDAFunctions.cuh:54-107 (mapParticles2Cells_CUDA, countingInCell_CUDA),
 // thrust::sort_by_key / gather / exclusive_scan.  The sort here is a
 // counting sort: integer atomics give each particle a slot in its cell, the
-// cell table is the exclusive scan of the histogram, and a per-cell sort by
-// old index then restores stability, so the permutation equals a stable
-// sort by cell id (what thrust's radix sort_by_key returns) on every run.
+// cell table is the exclusive scan of the histogram, and ranking each cell's
+// members by old index where they are consumed restores stability, so the
+// permutation equals a stable sort by cell id (what thrust's radix
+// sort_by_key returns) on every run.
 #include <hip/hip_runtime.h>
 
 #include "gg_device.hpp"
@@ -23,12 +24,10 @@ __global__ void __launch_bounds__(kBlock) k_hash_count(const float *__restrict__
                                                        DevGrid g, int *__restrict__ key,
                                                        int *__restrict__ slot,
                                                        int *__restrict__ count,
-                                                       int *__restrict__ ctr) {
+                                                       int *__restrict__ ctr,
+                                                       int *__restrict__ key_copy) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) {
-    ctr[0] = 0;                // big-cell counter of this build
-    ctr[kHugeCounter] = 0;     // cells for the multi-block path
-  }
+  if (i == 0) ctr[kHugeCounter] = 0;  // cells for the multi-block path
   // All lanes take part in the wave operations; lanes past n carry key -1.
   int c = -1;
   if (i < n) {
@@ -41,6 +40,7 @@ __global__ void __launch_bounds__(kBlock) k_hash_count(const float *__restrict__
       c = hash_cell(p3.x, p3.y, p3.z, g);
     }
     key[i] = c;
+    if (key_copy) key_copy[i] = c;
   }
   // Wave-aggregated slot reservation: each run of equal keys in adjacent
   // lanes (the input is the previous step's cell order, so runs are long)
@@ -62,46 +62,45 @@ __global__ void __launch_bounds__(kBlock) k_hash_count(const float *__restrict__
   if (i < n) slot[i] = basev + (lane - hl);
 }
 
-// Block sums of kScanTile-element tiles of count[0..m).
-__global__ void __launch_bounds__(kBlock) k_scan_reduce(const int *__restrict__ count, int m,
-                                                        int *__restrict__ part) {
-  __shared__ int wsum[kBlock / 64];
-  const int base = blockIdx.x * kScanTile + threadIdx.x * 8;
-  int s = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = base + k;
-    if (idx < m) s += count[idx];
-  }
-  s = wave_sum(s);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) wsum[wid] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-    for (int w = 0; w < kBlock / 64; ++w) t += wsum[w];
-    part[blockIdx.x] = t;
-  }
+// Words of the single-pass scan's tile states: a tile's sum, then its
+// inclusive prefix.  Read and written across XCDs by different blocks of one
+// launch: agent-scope atomics, one word each, so no fences.
+constexpr unsigned int kTileSum = 1u << 30, kTilePrefix = 2u << 30, kTileValue = kTileSum - 1u;
+__device__ __forceinline__ unsigned int tile_load(const unsigned int *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void tile_store(unsigned int *p, unsigned int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Exclusive scan of the (<= kScanMaxParts) partials in one block.
-__global__ void __launch_bounds__(1024) k_scan_parts(int *__restrict__ part, int np) {
-  __shared__ int buf[kScanMaxParts];
-  __shared__ int wtot[16];
-  const int t = threadIdx.x;
-  for (int k = t; k < np; k += 1024) buf[k] = part[k];
+// out[c] = sum of in[0..c) for c in [0, m] (totals below 2^30), in[] cleared
+// for the next build: one pass with decoupled look-back (Merrill and Garland
+// 2016).  A launch costs about 4 us here whatever it does, so this replaces a
+// reduce, a scan of the partial sums and an apply.  Tiles go to blocks in the
+// order the blocks start (sync[0]), so a tile only waits for tiles whose
+// blocks already run and publish their sums without waiting: every wait ends.
+// The last block to finish (sync[1]) leaves states and counters zero for the
+// next launch.  huge (optional): cells of more than kBigLds entries are
+// recorded as {cell, INT_MAX, 0} and found again through at_huge[cell].
+__global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
+                                                 unsigned int *__restrict__ state,
+                                                 int *__restrict__ sync, int *__restrict__ out,
+                                                 int *__restrict__ huge, int *__restrict__ at_huge,
+                                                 int *__restrict__ nhuge) {
+  __shared__ int tile_s, excl_s, last_s;
+  __shared__ int wtot[kBlock / 64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (threadIdx.x == 0) tile_s = atomicAdd(&sync[0], 1);
   __syncthreads();
-  // each thread owns 8 consecutive entries
-  const int b0 = t * 8;
+  const int tile = tile_s;
+  const int base = tile * kScanTile + threadIdx.x * 8;
   int loc[8];
   int s = 0;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    loc[k] = (b0 + k < np) ? buf[b0 + k] : 0;
+    loc[k] = base + k < m ? in[base + k] : 0;
     s += loc[k];
   }
-  // inclusive wave scan of per-thread sums
-  const int lane = t & 63, wid = t >> 6;
   int inc = s;
   for (int o = 1; o < 64; o <<= 1) {
     const int v = __shfl_up(inc, o, 64);
@@ -109,171 +108,142 @@ __global__ void __launch_bounds__(1024) k_scan_parts(int *__restrict__ part, int
   }
   if (lane == 63) wtot[wid] = inc;
   __syncthreads();
-  if (t == 0) {
-    int run = 0;
-    for (int w = 0; w < 16; ++w) {
-      const int v = wtot[w];
-      wtot[w] = run;
-      run += v;
+  int woff = 0, total = 0;
+  for (int w = 0; w < kBlock / 64; ++w) {
+    if (w < wid) woff += wtot[w];
+    total += wtot[w];
+  }
+  if (wid == 0) {
+    int excl = 0;
+    if (lane == 0)
+      tile_store(&state[tile], (unsigned int)total | (tile == 0 ? kTilePrefix : kTileSum));
+    // 64 tiles before this one at a time, back to the nearest prefix
+    for (int t0 = tile - 1; t0 >= 0; t0 -= 64) {
+      const int t = t0 - lane;
+      unsigned int v = t >= 0 ? tile_load(&state[t]) : kTilePrefix;
+      while (__any(v == 0u)) {
+        __builtin_amdgcn_s_sleep(1);
+        if (v == 0u) v = tile_load(&state[t]);
+      }
+      const unsigned long long pre = __ballot((v & kTilePrefix) != 0u);
+      const int upto = pre ? __ffsll((long long)pre) - 1 : 63;
+      excl += wave_sum(lane <= upto ? (int)(v & kTileValue) : 0);
+      if (pre) break;
+    }
+    if (lane == 0) {
+      if (tile > 0) tile_store(&state[tile], (unsigned int)(excl + total) | kTilePrefix);
+      excl_s = excl;
+      last_s = atomicAdd(&sync[1], 1) == (int)gridDim.x - 1;
     }
   }
   __syncthreads();
-  int run = wtot[wid] + inc - s;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    if (b0 + k < np) buf[b0 + k] = run;
-    run += loc[k];
-  }
-  __syncthreads();
-  for (int k = t; k < np; k += 1024) part[k] = buf[k];
-}
-
-// cell_start[c] = exclusive prefix of count; cell_start[m] = total.  Clears
-// count for the next build.
-__global__ void __launch_bounds__(kBlock) k_scan_apply(int *__restrict__ count, int m,
-                                                       const int *__restrict__ part,
-                                                       int *__restrict__ cell_start) {
-  __shared__ int wtot[kBlock / 64];
-  const int base = blockIdx.x * kScanTile + threadIdx.x * 8;
-  int loc[8];
-  int s = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = base + k;
-    loc[k] = idx < m ? count[idx] : 0;
-    s += loc[k];
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  int inc = s;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
-  if (lane == 63) wtot[wid] = inc;
-  __syncthreads();
-  int woff = 0;
-  for (int w = 0; w < wid; ++w) woff += wtot[w];
-  int run = part[blockIdx.x] + woff + inc - s;
+  int run = excl_s + woff + inc - s;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int idx = base + k;
     if (idx < m) {
-      cell_start[idx] = run;
-      count[idx] = 0;
-      if (idx == m - 1) cell_start[m] = run + loc[k];
+      out[idx] = run;
+      in[idx] = 0;
+      if (idx == m - 1) out[m] = run + loc[k];
+      if (huge && loc[k] > kBigLds) {
+        const int h = atomicAdd(nhuge, 1);
+        huge[3 * h] = idx;
+        huge[3 * h + 1] = 0x7fffffff;
+        huge[3 * h + 2] = 0;
+        at_huge[idx] = h;
+      }
     }
     run += loc[k];
   }
+  if (last_s) {
+    // every block has read the states it needs before it counted itself
+    for (int t = threadIdx.x; t < (int)gridDim.x; t += kBlock) tile_store(&state[t], 0u);
+    if (threadIdx.x < 2) sync[threadIdx.x] = 0;
+  }
 }
 
+// raw[cell_start + arrival slot] = i; for the cells recorded as huge also the
+// range [lo, hi) of their members' indices.
 __global__ void __launch_bounds__(kBlock) k_scatter(const int *__restrict__ key,
                                                     const int *__restrict__ slot, int n,
                                                     const int *__restrict__ cell_start,
-                                                    int *__restrict__ perm) {
+                                                    int *__restrict__ raw, int *__restrict__ huge,
+                                                    const int *__restrict__ at_huge) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int d = cell_start[key[i]] + slot[i];
-  if (d >= 0 && d < n) perm[d] = i;
+  int h = -1;
+  if (i < n) {
+    const int c = key[i];
+    const int s = cell_start[c];
+    const int d = s + slot[i];
+    if (d >= 0 && d < n) raw[d] = i;
+    if (huge && cell_start[c + 1] - s > kBigLds) h = at_huge[c];
+  }
+  // one pair of atomics per wave and huge cell (lanes are in index order)
+  const int lane = threadIdx.x & 63;
+  unsigned long long m = __ballot(h >= 0);
+  while (m) {
+    const int first = __ffsll((long long)m) - 1;
+    const unsigned long long mine = __ballot(h == __shfl(h, first, 64));
+    if (lane == first) {
+      atomicMin(&huge[3 * h + 1], i);
+      atomicMax(&huge[3 * h + 2], i + 64 - __clzll((long long)mine) - lane);
+    }
+    m &= ~mine;
+  }
 }
 
-// One thread per sorted slot d: raw[d] (the scatter's arrival order) goes
-// to cell_start[c] + (number of entries of its cell c with a smaller old
-// index), i.e. ascending old index within the cell.  Cells longer than
-// kSmallCell are copied as they are and queued (by their first slot) for
-// k_sort_big.
-__global__ void __launch_bounds__(kBlock) k_rank_small(const int *__restrict__ raw, int n,
-                                                       const int *__restrict__ key,
-                                                       const int *__restrict__ cell_start,
-                                                       int *__restrict__ perm,
-                                                       int *__restrict__ big,
-                                                       int *__restrict__ ctr) {
+// perm[slot of raw[d]] = raw[d]: a stable sort's permutation.
+__global__ void __launch_bounds__(kBlock) k_rank(const int *__restrict__ raw, int n,
+                                                 const int *__restrict__ key,
+                                                 const int *__restrict__ cell_start,
+                                                 int *__restrict__ perm) {
+  const int d = blockIdx.x * blockDim.x + threadIdx.x;
+  if (d >= n) return;
+  int c;
+  const int v = raw[d];
+  perm[sorted_slot(raw, key, cell_start, d, v, c)] = v;
+}
+
+// A set's payload permuted into the staging arrays (and back, in place, by
+// k_payload_back): one pass over all arrays where each had a gather and a
+// copy of its own.
+struct Payload {
+  gg_float3 *pos, *vel;
+  int *w[5];  // mass, is_animated, merge, merge_count, remove as words
+};
+__global__ void __launch_bounds__(kBlock)
+    k_rank_gather(const int *__restrict__ raw, int n, const int *__restrict__ key,
+                  const int *__restrict__ cell_start, Payload src, Payload tmp,
+                  int *__restrict__ p2c, int *__restrict__ perm_out) {
   const int d = blockIdx.x * blockDim.x + threadIdx.x;
   if (d >= n) return;
   const int v = raw[d];
-  const int c = key[v];
-  const int s = cell_start[c], e = cell_start[c + 1];
-  if (e - s > kSmallCell) {
-    perm[d] = v;
-    if (d == s) big[atomicAdd(&ctr[0], 1)] = c;
-    return;
-  }
-  int rank = 0;
-  for (int k = s; k < e; ++k) rank += raw[k] < v ? 1 : 0;
-  perm[s + rank] = v;
+  const gg_float3 x = src.pos[v];
+  gg_float3 u{};
+  int w[5];
+  if (src.vel) u = src.vel[v];
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    if (src.w[k]) w[k] = src.w[k][v];
+  int c;
+  const int o = sorted_slot(raw, key, cell_start, d, v, c);
+  tmp.pos[o] = x;
+  if (src.vel) tmp.vel[o] = u;
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    if (src.w[k]) tmp.w[k][o] = w[k];
+  if (p2c) p2c[o] = c;
+  if (perm_out) perm_out[o] = v;
 }
 
-// One block per queued cell (grid-stride over the queue).  Cells up to
-// kBigLds entries: bitonic sort of the old indices in LDS.  Larger cells
-// (e.g. the sentinel cell of particles outside the grid) go to the
-// multi-block path: the block records the cell and the range [lo, hi) of its
-// members' old indices in huge[] (k_huge_count / k_huge_write then compact
-// {i in [lo, hi) : key[i] == c} in index order over many blocks).
-__global__ void __launch_bounds__(kBlock) k_sort_big(const int *__restrict__ cell_start,
-                                                     int *__restrict__ perm,
-                                                     const int *__restrict__ big,
-                                                     int *__restrict__ ctr,
-                                                     int *__restrict__ huge) {
-  __shared__ int buf[kBigLds];
-  __shared__ int red[2][kBlock / 64];
-  const int nbig = ctr[0];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int b = blockIdx.x; b < nbig; b += gridDim.x) {
-    const int c = big[b];
-    const int s = cell_start[c], e = cell_start[c + 1];
-    const int len = e - s;
-    if (len <= kBigLds) {
-      int P = 1;
-      while (P < len) P <<= 1;
-      for (int k = threadIdx.x; k < P; k += blockDim.x) buf[k] = k < len ? perm[s + k] : 0x7fffffff;
-      __syncthreads();
-      for (int k = 2; k <= P; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-          for (int t = threadIdx.x; t < P; t += blockDim.x) {
-            const int u = t ^ j;
-            if (u > t) {
-              const int x = buf[t], y = buf[u];
-              const bool up = (t & k) == 0;
-              if ((x > y) == up) {
-                buf[t] = y;
-                buf[u] = x;
-              }
-            }
-          }
-          __syncthreads();
-        }
-      }
-      for (int k = threadIdx.x; k < len; k += blockDim.x) perm[s + k] = buf[k];
-      __syncthreads();
-    } else {
-      int lo = 0x7fffffff, hi = -1;
-      for (int k = s + threadIdx.x; k < e; k += blockDim.x) {
-        const int v = perm[k];
-        lo = v < lo ? v : lo;
-        hi = v > hi ? v : hi;
-      }
-      for (int o = 32; o > 0; o >>= 1) {
-        const int a = __shfl_xor(lo, o, 64), z = __shfl_xor(hi, o, 64);
-        lo = a < lo ? a : lo;
-        hi = z > hi ? z : hi;
-      }
-      if (lane == 0) {
-        red[0][wid] = lo;
-        red[1][wid] = hi;
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        for (int w = 1; w < kBlock / 64; ++w) {
-          lo = red[0][w] < lo ? red[0][w] : lo;
-          hi = red[1][w] > hi ? red[1][w] : hi;
-        }
-        const int h = atomicAdd(&ctr[kHugeCounter], 1);
-        huge[3 * h] = c;
-        huge[3 * h + 1] = lo;
-        huge[3 * h + 2] = hi + 1;
-      }
-      __syncthreads();
-    }
-  }
+__global__ void __launch_bounds__(kBlock) k_payload_back(int n, Payload dst, Payload tmp) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  dst.pos[i] = tmp.pos[i];
+  if (dst.vel) dst.vel[i] = tmp.vel[i];
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    if (dst.w[k]) dst.w[k][i] = tmp.w[k][i];
 }
 
 // Chunk p of kHugeChunks equal parts of [lo, hi).
@@ -318,7 +288,7 @@ __global__ void __launch_bounds__(kBlock) k_huge_write(const int *__restrict__ k
                                                        const int *__restrict__ ctr,
                                                        const int *__restrict__ huge,
                                                        const int *__restrict__ cnt,
-                                                       int *__restrict__ perm) {
+                                                       int *__restrict__ raw) {
   __shared__ int wcnt[kBlock / 64];
   const int nh = ctr[kHugeCounter];
   const int p = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -362,7 +332,7 @@ __global__ void __launch_bounds__(kBlock) k_huge_write(const int *__restrict__ k
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         if (m[q]) {
-          if (at < len) perm[s + at] = i0 + q;
+          if (at < len) raw[s + at] = i0 + q;
           ++at;
         }
       }
@@ -383,14 +353,6 @@ __global__ void __launch_bounds__(kBlock) k_gather_words(const uint32_t *__restr
   for (int w = 0; w < words; ++w) dst[(size_t)k * words + w] = src[(size_t)o * words + w];
 }
 
-__global__ void __launch_bounds__(kBlock) k_gather_keys(const int *__restrict__ key,
-                                                        const int *__restrict__ perm, int n,
-                                                        int *__restrict__ out) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  out[k] = key[perm[k]];
-}
-
 __global__ void __launch_bounds__(kBlock) k_pack_boundary(const float *__restrict__ pos, int n,
                                                           float rb, float4 *__restrict__ out) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -400,10 +362,23 @@ __global__ void __launch_bounds__(kBlock) k_pack_boundary(const float *__restric
 
 static inline int blocks_for(long long n) { return (int)((n + kBlock - 1) / kBlock); }
 
-// Hash (or the given keys), counting sort, cell table and perm for `n`
-// particles.
+static int launch_scan(int *in, int m, int *out, const gg_workspace *ws, int *huge, int *at_huge,
+                       int *nhuge, hipStream_t st) {
+  Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
+                         ws->bmax);
+  const int np = (m + kScanTile - 1) / kScanTile;
+  k_scan<<<np, kBlock, 0, st>>>(in, m, at<unsigned int>(ws, L.part),
+                                at<int>(ws, L.ctr2) + kScanSync, out, huge, at_huge, nhuge);
+  GG_LAUNCH_CHECK();
+  return GG_OK;
+}
+
+// Hash (or the given keys), counting sort and cell table for n particles:
+// the workspace's itmp array ends with each cell's members (ascending in
+// cells of more than kBigLds, in any order below that: sorted_slot ranks
+// them where they are consumed).
 int sort_by_cell_keys(const float *pos, const int *keys_in, int n, int *cell_start,
-                      const gg_workspace *ws, hipStream_t st) {
+                      const gg_workspace *ws, hipStream_t st, int *key_copy) {
   Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
                          ws->bmax);
   const DevGrid g = dev_grid(ws->grid);
@@ -411,38 +386,26 @@ int sort_by_cell_keys(const float *pos, const int *keys_in, int n, int *cell_sta
   int *count = at<int>(ws, L.count);
   int *key = at<int>(ws, L.key);
   int *slot = at<int>(ws, L.slot);
-  int *perm = at<int>(ws, L.perm);
-  int *part = at<int>(ws, L.part);
-  int *big = at<int>(ws, L.big);
+  int *raw = at<int>(ws, L.itmp);
+  int *at_huge = at<int>(ws, L.big);
   int *ctr = at<int>(ws, L.ctr);
+  // the huge-cell records and per-chunk counts live in the permutation's
+  // array, which is written after the sort: (3 + kHugeChunks) ints per cell
+  // of more than kBigLds particles (at most n / kBigLds of them)
+  int *huge = n > kBigLds ? at<int>(ws, L.perm) : nullptr;
+  int *hcnt = at<int>(ws, L.perm) + 3 * (n / kBigLds + 1);
   const int nb = n > 0 ? blocks_for(n) : 1;
-  k_hash_count<<<nb, kBlock, 0, st>>>(pos, keys_in, n, g, key, slot, count, ctr);
+  k_hash_count<<<nb, kBlock, 0, st>>>(pos, keys_in, n, g, key, slot, count, ctr, key_copy);
   GG_LAUNCH_CHECK();
-  const int np = (m + kScanTile - 1) / kScanTile;
-  k_scan_reduce<<<np, kBlock, 0, st>>>(count, m, part);
-  GG_LAUNCH_CHECK();
-  k_scan_parts<<<1, 1024, 0, st>>>(part, np);
-  GG_LAUNCH_CHECK();
-  k_scan_apply<<<np, kBlock, 0, st>>>(count, m, part, cell_start);
-  GG_LAUNCH_CHECK();
+  GG_TRY(launch_scan(count, m, cell_start, ws, huge, at_huge, ctr + kHugeCounter, st));
   if (n > 0) {
-    int *raw = at<int>(ws, L.itmp);
-    k_scatter<<<blocks_for(n), kBlock, 0, st>>>(key, slot, n, cell_start, raw);
-    GG_LAUNCH_CHECK();
-    k_rank_small<<<blocks_for(n), kBlock, 0, st>>>(raw, n, key, cell_start, perm, big, ctr);
+    k_scatter<<<nb, kBlock, 0, st>>>(key, slot, n, cell_start, raw, huge, at_huge);
     GG_LAUNCH_CHECK();
   }
-  // the huge-cell records and per-chunk counts live in the arrival-slot
-  // array, which nothing reads after the scatter: (3 + kHugeChunks) ints per
-  // cell of more than kBigLds particles (at most n / kBigLds of them)
-  int *huge = slot;
-  int *hcnt = slot + 3 * (n / kBigLds + 1);
-  k_sort_big<<<256, kBlock, 0, st>>>(cell_start, perm, big, ctr, huge);
-  GG_LAUNCH_CHECK();
-  if (n > kBigLds) {
+  if (huge) {
     k_huge_count<<<kHugeChunks, kBlock, 0, st>>>(key, ctr, huge, hcnt);
     GG_LAUNCH_CHECK();
-    k_huge_write<<<kHugeChunks, kBlock, 0, st>>>(key, cell_start, ctr, huge, hcnt, perm);
+    k_huge_write<<<kHugeChunks, kBlock, 0, st>>>(key, cell_start, ctr, huge, hcnt, raw);
     GG_LAUNCH_CHECK();
   }
   return GG_OK;
@@ -453,22 +416,23 @@ int sort_by_cell(const float *pos, int n, int *cell_start, const gg_workspace *w
   return sort_by_cell_keys(pos, nullptr, n, cell_start, ws, st);
 }
 
+// perm of the sort just done.
+int sort_permutation(int n, const int *cell_start, const gg_workspace *ws, hipStream_t st) {
+  if (n <= 0) return GG_OK;
+  Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
+                         ws->bmax);
+  k_rank<<<blocks_for(n), kBlock, 0, st>>>(at<int>(ws, L.itmp), n, at<int>(ws, L.key), cell_start,
+                                           at<int>(ws, L.perm));
+  GG_LAUNCH_CHECK();
+  return GG_OK;
+}
+
 // out[k] = sum of in[0..k) for k in [0, m], in[] cleared.  m <= kScanTile *
-// kScanMaxParts (the workspace's partials array holds the tile sums).
+// kScanMaxParts (the workspace holds a state per tile).
 int scan_exclusive(int *in, int m, int *out, const gg_workspace *ws, hipStream_t st) {
   if (m <= 0) return GG_OK;
   if ((long long)m > (long long)kScanTile * kScanMaxParts) return GG_ERR_CAPACITY;
-  Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
-                         ws->bmax);
-  int *part = at<int>(ws, L.part);
-  const int np = (m + kScanTile - 1) / kScanTile;
-  k_scan_reduce<<<np, kBlock, 0, st>>>(in, m, part);
-  GG_LAUNCH_CHECK();
-  k_scan_parts<<<1, 1024, 0, st>>>(part, np);
-  GG_LAUNCH_CHECK();
-  k_scan_apply<<<np, kBlock, 0, st>>>(in, m, part, out);
-  GG_LAUNCH_CHECK();
-  return GG_OK;
+  return launch_scan(in, m, out, ws, nullptr, nullptr, nullptr, st);
 }
 
 int gather_inplace(void *arr, int words, const int *perm, int n, void *tmp, hipStream_t st) {
@@ -482,7 +446,7 @@ int gather_inplace(void *arr, int words, const int *perm, int n, void *tmp, hipS
 
 int grid_build_general(gg_particles *set, gg_adaptive *ad, int *cell_start, int *perm_out,
                        const gg_workspace *ws, hipStream_t st, int capacity_limit,
-                       const int *keys) {
+                       const int *keys, int *key_copy) {
   if (!set || !cell_start) return GG_ERR_INVALID;
   GG_TRY(check_ws(ws));
   const int n = set->n;
@@ -492,28 +456,23 @@ int grid_build_general(gg_particles *set, gg_adaptive *ad, int *cell_start, int 
   Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
                          ws->bmax);
   GG_TRY(sort_by_cell_keys(reinterpret_cast<const float *>(set->pos), keys, n, cell_start, ws,
-                           st));
-  const int *perm = at<int>(ws, L.perm);
-  const int *key = at<int>(ws, L.key);
+                           st, key_copy));
   if (n == 0) return GG_OK;
-  void *t3 = at<void>(ws, L.v3tmp0);
-  void *t1 = at<void>(ws, L.itmp0);
-  GG_TRY(gather_inplace(set->pos, 3, perm, n, t3, st));
-  GG_TRY(gather_inplace(set->vel, 3, perm, n, t3, st));
-  GG_TRY(gather_inplace(set->mass, 1, perm, n, t1, st));
-  GG_TRY(gather_inplace(set->is_animated, 1, perm, n, t1, st));
-  if (ad) {
-    GG_TRY(gather_inplace(ad->merge, 1, perm, n, t1, st));
-    GG_TRY(gather_inplace(ad->merge_count, 1, perm, n, t1, st));
-    GG_TRY(gather_inplace(ad->remove, 1, perm, n, t1, st));
-  }
-  if (set->particle_2_cell) {
-    k_gather_keys<<<blocks_for(n), kBlock, 0, st>>>(key, perm, n, set->particle_2_cell);
-    GG_LAUNCH_CHECK();
-  }
-  if (perm_out)
-    GG_TRY(hip_status(
-        hipMemcpyAsync(perm_out, perm, (size_t)n * 4, hipMemcpyDeviceToDevice, st)));
+  const Payload p{set->pos,
+                  set->vel,
+                  {reinterpret_cast<int *>(set->mass), set->is_animated,
+                   ad ? reinterpret_cast<int *>(ad->merge) : nullptr,
+                   ad ? ad->merge_count : nullptr, ad ? ad->remove : nullptr}};
+  const Payload t{at<gg_float3>(ws, L.v3tmp0),
+                  at<gg_float3>(ws, L.v3tmp1),
+                  {at<int>(ws, L.ftmp0), at<int>(ws, L.itmp0), at<int>(ws, L.ftmp1),
+                   at<int>(ws, L.itmp1), at<int>(ws, L.itmp2)}};
+  k_rank_gather<<<blocks_for(n), kBlock, 0, st>>>(at<int>(ws, L.itmp), n, at<int>(ws, L.key),
+                                                  cell_start, p, t, set->particle_2_cell,
+                                                  perm_out);
+  GG_LAUNCH_CHECK();
+  k_payload_back<<<blocks_for(n), kBlock, 0, st>>>(n, p, t);
+  GG_LAUNCH_CHECK();
   return GG_OK;
 }
 

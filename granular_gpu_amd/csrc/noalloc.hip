@@ -82,10 +82,12 @@ extern "C" int gg_step_noalloc(gg_particles *set, gg_adaptive *ad, int *cell_sta
   ws.base = base;
   ws.bytes = kScratchBytes;
   GG_TRY(check_ws(&ws));
-  // zero what the step expects at zero: the cell histogram and the counters
+  // zero what the step expects at zero: the cell histogram, the scan's states
+  // and the counters
   const Layout L = make_layout(ws.capacity, ws.boundary_capacity, grid, ws.max_sweeps, ws.gmax,
                                ws.bmax);
   GG_TRY(gg_fill_u32(at<void>(&ws, L.count), (size_t)grid_cells(grid) + 1, 0u, stream));
+  GG_TRY(gg_fill_u32(at<void>(&ws, L.part), (L.big - L.part) / 4, 0u, stream));
   GG_TRY(gg_fill_u32(at<void>(&ws, L.ctr), 64, 0u, stream));
   GG_TRY(gg_fill_u32(at<void>(&ws, L.ctr2), 64, 0u, stream));
   GG_TRY(gg_fill_u32(at<void>(&ws, L.fbqc), 2, 0u, stream));

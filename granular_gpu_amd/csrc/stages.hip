@@ -92,5 +92,6 @@ extern "C" int gg_sort_positions_by_key(gg_particles *set, int *cell_start,
   Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
                          ws->bmax);
   GG_TRY(sort_by_cell_keys(nullptr, set->particle_2_cell, set->n, cell_start, ws, stream));
+  GG_TRY(sort_permutation(set->n, cell_start, ws, stream));
   return gather_inplace(set->pos, 3, at<int>(ws, L.perm), set->n, at<void>(ws, L.v3tmp0), stream);
 }

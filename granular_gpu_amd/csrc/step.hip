@@ -56,8 +56,8 @@ __device__ __forceinline__ uint2 quantise(const float4 &x, float per_unit) {
 }
 
 __global__ void __launch_bounds__(kBlock)
-    k_permute_predict(int n, const int *__restrict__ perm, const int *__restrict__ key,
-                      const float *__restrict__ pos, const float *__restrict__ vel,
+    k_permute_predict(int n, const int *__restrict__ raw, const int *__restrict__ key,
+                      const int *__restrict__ cell_start, const float *__restrict__ pos, const float *__restrict__ vel,
                       const float *__restrict__ mass, float4 *__restrict__ x0,
                       float4 *__restrict__ off0, float4 *__restrict__ d0,
                       float4 *__restrict__ xs,
@@ -69,13 +69,13 @@ __global__ void __launch_bounds__(kBlock)
                       double denom, int *__restrict__ dirty, int ndirty,
                       int *__restrict__ fbcount, int *__restrict__ fbq_len,
                       unsigned int *__restrict__ bpart, uint2 *__restrict__ xq, float per_unit) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int k = i; k < ndirty; k += gridDim.x * blockDim.x) dirty[k] = 0;
-  if (i < kFallbackSlots) fbcount[i] = 0;
-  if (i < 2) fbq_len[i] = 0;
+  const int d = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int k = d; k < ndirty; k += gridDim.x * blockDim.x) dirty[k] = 0;
+  if (d < kFallbackSlots) fbcount[d] = 0;
+  if (d < 2) fbq_len[d] = 0;
   float dmax = 0.0f, rmax = 0.0f;
-  if (i < n) {
-    const int o = perm ? perm[i] : i;
+  if (d < n) {
+    const int o = raw ? raw[d] : d;
     const Packed3 p3 = ld3(pos, o), v3 = ld3(vel, o);
     const float px = p3.x, py = p3.y, pz = p3.z;
     float vx = v3.x, vy = v3.y, vz = v3.z;
@@ -85,6 +85,9 @@ __global__ void __launch_bounds__(kBlock)
     const float Dx = dt * vx, Dy = dt * vy, Dz = dt * vz;
     const float m = mass[o];
     const float r = radius_contact(m, denom);
+    // o's place in the stable order (identity without a sort)
+    int i = d, c = 0;
+    if (raw) i = sorted_slot(raw, key, cell_start, d, o, c);
     x0[i] = make_float4(px, py, pz, r);
     off0[i] = make_float4(Dx, Dy, Dz, 0.0f);
     d0[i] = make_float4(Dx, Dy, Dz, 0.0f);
@@ -93,7 +96,7 @@ __global__ void __launch_bounds__(kBlock)
     xq[i] = quantise(x, per_unit);
     mass_tmp[i] = m;
     if (ms_out) ms_out[i] = m * exp_f(-py);
-    if (perm && p2c) p2c[i] = key[o];
+    if (raw && p2c) p2c[i] = c;
     if (rem_in) rem_tmp[i] = rem_in[o];
     if (mer_in) mer_tmp[i] = mer_in[o];
     if (mc_in) mc_tmp[i] = mc_in[o];
@@ -101,8 +104,8 @@ __global__ void __launch_bounds__(kBlock)
     if (!(Dx == Dx && Dy == Dy && Dz == Dz)) dmax = __builtin_inff();
     rmax = r == r ? r : __builtin_inff();
   }
-  // per-block largest |D| component and radius; k_reduce_bounds folds the
-  // blocks
+  // per-block largest |D| component and radius; the list build's first block
+  // folds the blocks
   __shared__ float red[2][kBlock / 64];
   const float wd = wave_max(dmax);
   const float wr = wave_max(rmax);
@@ -123,12 +126,13 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // bounds[0..1] = maxima of the nb per-block values (non-negative floats
-// order like their bit patterns).  One block.
-__global__ void __launch_bounds__(1024) k_reduce_bounds(const unsigned int *__restrict__ bpart,
-                                                        int nb, unsigned int *__restrict__ bounds) {
-  __shared__ unsigned int red[2][16];
+// order like their bit patterns), by one wave.
+__device__ __forceinline__ void reduce_bounds(const unsigned int *__restrict__ bpart, int nb,
+                                              unsigned int *__restrict__ bounds) {
+  const int lane = threadIdx.x & 63;
   unsigned int a = 0u, b = 0u;
-  for (int k = threadIdx.x; k < nb; k += 1024) {
+#pragma unroll 8
+  for (int k = lane; k < nb; k += 64) {
     a = max(a, bpart[2 * k]);
     b = max(b, bpart[2 * k + 1]);
   }
@@ -136,16 +140,7 @@ __global__ void __launch_bounds__(1024) k_reduce_bounds(const unsigned int *__re
     a = max(a, (unsigned int)__shfl_xor((int)a, o, 64));
     b = max(b, (unsigned int)__shfl_xor((int)b, o, 64));
   }
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = a;
-    red[1][threadIdx.x >> 6] = b;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 0; w < 16; ++w) {
-      a = max(a, red[0][w]);
-      b = max(b, red[1][w]);
-    }
+  if (lane == 0) {
     bounds[0] = a;
     bounds[1] = b;
   }
@@ -185,6 +180,11 @@ struct ListArgs {
   int remap;
   SceneView sv;
   RefreshGate gate;
+  // predict's per-block maxima, reduced into bounds by the launch's first
+  // block (nothing else in it reads them); null: no such block
+  const unsigned int *__restrict__ bpart;
+  int nbpart;
+  unsigned int *__restrict__ bounds;
 };
 
 // Boundary candidates of i in scan order.
@@ -228,7 +228,13 @@ template <int BS, bool SCENES>
 __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
   if (!gate_open(a.gate)) return;
   __shared__ int queue[BS / 64][kListChunk][64];
-  const int i = xcd_block(blockIdx.x, gridDim.x, a.remap) * blockDim.x + threadIdx.x;
+  const int extra = a.bpart ? 1 : 0;
+  if (extra && blockIdx.x == 0) {
+    if (threadIdx.x < 64) reduce_bounds(a.bpart, a.nbpart, a.bounds);
+    return;
+  }
+  const int i = xcd_block(blockIdx.x - extra, gridDim.x - extra, a.remap) * blockDim.x +
+                threadIdx.x;
   int(*const q)[64] = queue[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63;
   const bool live = i < a.n;
@@ -343,8 +349,13 @@ constexpr int kWideListMax = 65536;
 template <bool SCENES>
 __global__ void __launch_bounds__(64) k_nlist_wide(ListArgs a) {
   if (!gate_open(a.gate)) return;
+  const int extra = a.bpart ? 1 : 0;
+  if (extra && blockIdx.x == 0) {
+    reduce_bounds(a.bpart, a.nbpart, a.bounds);
+    return;
+  }
   const int lane = threadIdx.x & 63, sub = lane & 15, grp = lane & 48;
-  const int ib = 4 * xcd_block(blockIdx.x, gridDim.x, a.remap) + (lane >> 4);
+  const int ib = 4 * xcd_block(blockIdx.x - extra, gridDim.x - extra, a.remap) + (lane >> 4);
   const bool live = ib < a.n;
   const int i = live ? ib : 0;
   const LocalGrid lg = local_grid<SCENES>(a.sv, i, a.g, a.sc);
@@ -1085,7 +1096,7 @@ static SweepConst sweep_const(const gg_params *p, const gg_workspace *ws) {
 
 template <int BS, bool SCENES>
 static int launch_nlist_bs(const ListArgs &a, hipStream_t st) {
-  k_nlist<BS, SCENES><<<(a.n + BS - 1) / BS, BS, 0, st>>>(a);
+  k_nlist<BS, SCENES><<<(a.n + BS - 1) / BS + (a.bpart ? 1 : 0), BS, 0, st>>>(a);
   GG_LAUNCH_CHECK();
   return GG_OK;
 }
@@ -1104,11 +1115,12 @@ static float quant_per_unit(const gg_workspace *ws) {
   return (float)kQuantUnits / ws->grid.cell_length;
 }
 
-// The lists of n particles at positions xs (xq: the same, quantised).  near:
+// The lists of n particles at positions xs (xq: the same, quantised).
+// nbpart > 0: also reduce that many of predict's per-block bounds.  near:
 // whether the near lists are built, in the adaptive passes' arrays (no
 // adaptive pass may run between this and the sweeps that read them).
 static int launch_nlist(int n, const float4 *xs, const int *cs, const int *bcs,
-                        const gg_params *p, const gg_workspace *ws, bool near,
+                        const gg_params *p, const gg_workspace *ws, bool near, int nbpart,
                         const SceneView *sv, hipStream_t st,
                         RefreshGate gate = RefreshGate{nullptr, nullptr, 0}) {
   Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
@@ -1136,9 +1148,12 @@ static int launch_nlist(int n, const float4 *xs, const int *cs, const int *bcs,
   a.remap = (p->flags & GG_FLAG_NO_XCD_REMAP) ? 0 : 1;
   a.sv = sv ? *sv : SceneView{nullptr, nullptr, 0};
   a.gate = gate;
+  a.bpart = nbpart > 0 ? at<unsigned int>(ws, L.bpart) : nullptr;
+  a.nbpart = nbpart;
+  a.bounds = at<unsigned int>(ws, L.bounds);
   // (a block size asked for is k_nlist's; results do not depend on either)
   if (n <= kWideListMax && p->nlist_block == 0) {
-    const int blocks = (n + 3) / 4;
+    const int blocks = (n + 3) / 4 + (a.bpart ? 1 : 0);
     if (sv)
       k_nlist_wide<true><<<blocks, 64, 0, st>>>(a);
     else
@@ -1150,9 +1165,9 @@ static int launch_nlist(int n, const float4 *xs, const int *cs, const int *bcs,
   return sv ? launch_nlist_sc<true>(bs, a, st) : launch_nlist_sc<false>(bs, a, st);
 }
 
-// permute (perm may be null = identity) + predict + lists.  sv: scenes
-// sharing the set (null: one scene).
-static int run_predict(gg_particles *set, gg_adaptive *ad, const int *perm, const int *key,
+// permute (raw: the sort's cell members; null = identity) + predict + lists.
+// sv: scenes sharing the set (null: one scene).
+static int run_predict(gg_particles *set, gg_adaptive *ad, const int *raw, const int *key,
                        const int *cs, const int *bcs, int nbnd, const gg_params *p,
                        const gg_workspace *ws, hipStream_t st, bool near,
                        const SceneView *sv = nullptr) {
@@ -1165,7 +1180,7 @@ static int run_predict(gg_particles *set, gg_adaptive *ad, const int *perm, cons
   const int nblk = n > 0 ? blocks_for(n) : 1;
   prof_begin(GG_STAGE_PREDICT, st);
   k_permute_predict<<<nblk, kBlock, 0, st>>>(
-      n, perm, key, reinterpret_cast<const float *>(set->pos),
+      n, raw, key, cs, reinterpret_cast<const float *>(set->pos),
       reinterpret_cast<const float *>(set->vel), set->mass, at<float4>(ws, L.x0),
       at<float4>(ws, L.off0), at<float4>(ws, L.d0), at<float4>(ws, L.off1), at<float>(ws, L.ftmp0),
       set->scaled_mass,
@@ -1175,13 +1190,10 @@ static int run_predict(gg_particles *set, gg_adaptive *ad, const int *perm, cons
       at<int>(ws, L.ctr) + 1, at<int>(ws, L.fbqc), at<unsigned int>(ws, L.bpart),
       at<uint2>(ws, L.v3tmp0), quant_per_unit(ws));
   GG_LAUNCH_CHECK();
-  k_reduce_bounds<<<1, 1024, 0, st>>>(at<unsigned int>(ws, L.bpart), nblk,
-                                      at<unsigned int>(ws, L.bounds));
-  GG_LAUNCH_CHECK();
   prof_end(GG_STAGE_PREDICT, st);
   if (lists_on(p, ws) && n > 0) {
     prof_begin(GG_STAGE_NLIST, st);
-    GG_TRY(launch_nlist(n, at<float4>(ws, L.off1), cs, bcs, p, ws, near, sv, st));
+    GG_TRY(launch_nlist(n, at<float4>(ws, L.off1), cs, bcs, p, ws, near, nblk, sv, st));
     prof_end(GG_STAGE_NLIST, st);
   }
   (void)nbnd;
@@ -1333,7 +1345,7 @@ static int run_refresh(const gg_particles *set, const int *cs, const int *bcs,
                                                     at<uint2>(ws, L.v3tmp0), quant_per_unit(ws),
                                                     gate);
   GG_LAUNCH_CHECK();
-  GG_TRY(launch_nlist(n, xs, cs, bcs, p, ws, true, sv, st, gate));
+  GG_TRY(launch_nlist(n, xs, cs, bcs, p, ws, true, 0, sv, st, gate));
   prof_end(GG_STAGE_NLIST, st);
   return GG_OK;
 }
@@ -1396,7 +1408,7 @@ extern "C" int gg_step(gg_particles *set, gg_adaptive *ad, int *cell_start,
   prof_begin(GG_STAGE_SORT, stream);
   GG_TRY(sort_by_cell(reinterpret_cast<const float *>(set->pos), set->n, cell_start, ws, stream));
   prof_end(GG_STAGE_SORT, stream);
-  GG_TRY(run_predict(set, ad, at<int>(ws, L.perm), at<int>(ws, L.key), cell_start, bcell_start,
+  GG_TRY(run_predict(set, ad, at<int>(ws, L.itmp), at<int>(ws, L.key), cell_start, bcell_start,
                      boundary->n, params, ws, stream, true));
   const int K = params->stab_iters + params->solver_iters;
   for (int k = 0; k < K; ++k) {
@@ -1428,7 +1440,7 @@ extern "C" int gg_step_scenes(gg_particles *set, int *cell_start, const gg_parti
   GG_TRY(sort_by_cell_keys(reinterpret_cast<const float *>(set->pos), keys, set->n, cell_start,
                            ws, stream));
   prof_end(GG_STAGE_SORT, stream);
-  GG_TRY(run_predict(set, nullptr, at<int>(ws, L.perm), at<int>(ws, L.key), cell_start,
+  GG_TRY(run_predict(set, nullptr, at<int>(ws, L.itmp), at<int>(ws, L.key), cell_start,
                      bcell_start, boundary->n, params, ws, stream, true, &sv));
   const int K = params->stab_iters + params->solver_iters;
   for (int k = 0; k < K; ++k) {

@@ -36,12 +36,6 @@ __global__ void __launch_bounds__(kBlock)
   fvel[3 * i + 2] = vz;
 }
 
-__global__ void __launch_bounds__(kBlock) k_copy_int(const int *__restrict__ src,
-                                                     int *__restrict__ dst, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-
 static inline int blocks_for(long long n) { return (int)((n + kBlock - 1) / kBlock); }
 
 }  // namespace gg
@@ -80,14 +74,7 @@ extern "C" int gg_upsampled_sort(gg_particles *fine, int *fine_cell_start,
   tmp.mass = nullptr;
   tmp.is_animated = nullptr;
   GG_TRY(grid_build_general(&tmp, nullptr, fine_cell_start, nullptr, fine_ws, stream,
-                            fine_ws->capacity));
-  if (p2c && fine->n > 0) {
-    Layout L = make_layout(fine_ws->capacity, fine_ws->boundary_capacity, fine_ws->grid,
-                           fine_ws->max_sweeps, fine_ws->gmax, fine_ws->bmax);
-    k_copy_int<<<blocks_for(fine->n), kBlock, 0, stream>>>(at<int>(fine_ws, L.key), p2c,
-                                                           fine->n);
-    GG_LAUNCH_CHECK();
-  }
+                            fine_ws->capacity, nullptr, p2c));
   prof_end(GG_STAGE_UPSAMPLE_SORT, stream);
   return GG_OK;
 }
