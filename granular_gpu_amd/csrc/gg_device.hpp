@@ -366,8 +366,8 @@ __device__ __forceinline__ bool granular_terms(const float4 &bi, const float4 &o
 constexpr unsigned int kSqrtFastMinBits = 0x0f800000u;  // 2^-96
 template <bool FRIC, bool STRICT>
 __device__ __forceinline__ bool fast_terms(float px, float py, float pz, float rx, float ry,
-                                           float rz, float rc, float mu_s, float mu_k, float3 &a,
-                                           bool &redo) {
+                                           float rz, float rc, float mu_s, float mu_k, float3 &c,
+                                           float3 &f, bool &redo) {
   const float d2 = px * px + py * py + pz * pz;
   float y;
   const float d = sqrt_rsq(d2, y);
@@ -377,9 +377,7 @@ __device__ __forceinline__ bool fast_terms(float px, float py, float pz, float r
   const float inv = rcp_refine(d, y, redo);
   const float delta = rc - d;
   const float s = delta * inv;
-  a.x = a.x + s * px;
-  a.y = a.y + s * py;
-  a.z = a.z + s * pz;
+  c = make_float3(s * px, s * py, s * pz);
   if (FRIC) {
     const float nx = px * inv, ny = py * inv, nz = pz * inv;
     const float rn = rx * nx + ry * ny + rz * nz;
@@ -390,12 +388,10 @@ __device__ __forceinline__ bool fast_terms(float px, float py, float pz, float r
     const bool fixed = tl2 < fmaxf(lim * lim, 1.401298464e-45f);
     float yt;
     const float dt = sqrt_rsq(tl2, yt);
-    const float c = fminf(div_by(mu_k * delta, dt, rcp_refine(dt, yt, redo)), 1.0f);
+    const float q = fminf(div_by(mu_k * delta, dt, rcp_refine(dt, yt, redo)), 1.0f);
     redo |= !fixed && __float_as_uint(tl2) - kSqrtFastMinBits > 0x53800000u - kSqrtFastMinBits;
-    const float f = fixed ? 1.0f : c;
-    a.x = a.x - tx * f;
-    a.y = a.y - ty * f;
-    a.z = a.z - tz * f;
+    const float k = fixed ? 1.0f : q;
+    f = make_float3(tx * k, ty * k, tz * k);
   }
   return true;
 }

@@ -87,12 +87,13 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
                                                  int *__restrict__ sync, int *__restrict__ out,
                                                  int *__restrict__ huge, int *__restrict__ at_huge,
                                                  int *__restrict__ nhuge) {
-  __shared__ int tile_s, excl_s, last_s;
+  __shared__ int tile_s, excl_s;
   __shared__ int wtot[kBlock / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (threadIdx.x == 0) tile_s = atomicAdd(&sync[0], 1);
+  const bool alone = gridDim.x == 1;  // one tile: nothing to exchange
+  if (!alone && threadIdx.x == 0) tile_s = atomicAdd(&sync[0], 1);
   __syncthreads();
-  const int tile = tile_s;
+  const int tile = alone ? 0 : tile_s;
   const int base = tile * kScanTile + threadIdx.x * 8;
   int loc[8];
   int s = 0;
@@ -113,7 +114,9 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
     if (w < wid) woff += wtot[w];
     total += wtot[w];
   }
-  if (wid == 0) {
+  if (alone) {
+    if (threadIdx.x == 0) excl_s = 0;
+  } else if (wid == 0) {
     int excl = 0;
     if (lane == 0)
       tile_store(&state[tile], (unsigned int)total | (tile == 0 ? kTilePrefix : kTileSum));
@@ -133,7 +136,6 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
     if (lane == 0) {
       if (tile > 0) tile_store(&state[tile], (unsigned int)(excl + total) | kTilePrefix);
       excl_s = excl;
-      last_s = atomicAdd(&sync[1], 1) == (int)gridDim.x - 1;
     }
   }
   __syncthreads();
@@ -155,10 +157,14 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
     }
     run += loc[k];
   }
-  if (last_s) {
-    // every block has read the states it needs before it counted itself
-    for (int t = threadIdx.x; t < (int)gridDim.x; t += kBlock) tile_store(&state[t], 0u);
-    if (threadIdx.x < 2) sync[threadIdx.x] = 0;
+  if (!alone && wid == 0) {
+    // every block has read the states it needs before it counts itself
+    int done = 0;
+    if (lane == 0) done = atomicAdd(&sync[1], 1);
+    if (__shfl(done, 0, 64) == (int)gridDim.x - 1) {
+      for (int t = lane; t < (int)gridDim.x; t += 64) tile_store(&state[t], 0u);
+      if (lane < 2) sync[lane] = 0;
+    }
   }
 }
 
