@@ -50,7 +50,8 @@ constexpr int kFallbackSlots = 62;  // ctr[1 + k % 62] = full-stencil count of s
 // scan against 0.15 ns per particle of a build at 4M particles)
 constexpr int kRefreshCost = 8;
 // ctr[63..] are not used by the sweeps; the adaptive passes use ctr2 (own region)
-constexpr int kMergeRounds = 12;    // parallel claim-resolution rounds before the finisher
+constexpr int kMergeRounds = 10;    // launched claim-resolution rounds before the finisher,
+constexpr int kMergeSet = 131072;   // for sets up to this
 
 // Byte offsets of every buffer inside the caller's workspace.  Every region
 // starts on a 256-byte boundary.

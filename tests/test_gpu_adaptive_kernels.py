@@ -1,0 +1,107 @@
+"""GPU tests of the 16-lane stencil passes and of the claim finisher where
+they can go wrong: few particles, more neighbours than the scan's list holds,
+radii of several sizes, and chains of claims as long as a set, in the
+finisher's on-chip and its global form; all against the oracle bit for bit."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from granular_gpu_amd import scenes
+from oracle import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(pos, mass, cells):
+    n = pos.shape[0]
+    L = float(scenes.CELL_LENGTH)
+    return scenes.Scene(name="t", pos=pos.astype(np.float32), vel=np.zeros((n, 3), np.float32),
+                        mass=mass.astype(np.float32), boundary=np.zeros((1, 3), np.float32) + 0.01,
+                        space=tuple(L * c for c in cells), cell_length=scenes.CELL_LENGTH,
+                        cells=cells, dt=np.float32(0.002), gravity=(0.0, -9.8, 0.0),
+                        density=scenes.DENSITY_R001, radius=0.01)
+
+
+def _cloud(n, seed, crowd):
+    rng = np.random.default_rng(seed)
+    cells = (6, 5, 7)
+    pos = rng.random((n, 3)) * (np.array(cells) * float(scenes.CELL_LENGTH))
+    pos[: int(crowd * n)] = 0.1 + 0.06 * rng.random((int(crowd * n), 3))
+    return _scene(pos, rng.choice([0.125, 1.0, 2.0, 8.0], n), cells)
+
+
+def _lines(lines, length):
+    # cand[i] = i + 1 along each line: every claim waits for the one before
+    z = 0.02 + 0.03 * np.arange(length)
+    pos = np.concatenate([np.stack([np.full(length, 0.02 + 0.05 * k), np.full(length, 0.02), z], 1)
+                          for k in range(lines)])
+    L = float(scenes.CELL_LENGTH)
+    cells = (int(0.05 * lines / L) + 2, 1, int(z[-1] / L) + 2)
+    return _scene(pos, np.ones(pos.shape[0]), cells)
+
+
+def _sorted_sim(s):
+    from granular_gpu_amd.device import AdaptiveSim
+    sim = AdaptiveSim(s)
+    sim.grid_build()
+    torch.cuda.synchronize()
+    n = sim.n
+    g = lambda t: t[:n].cpu().numpy().copy()
+    return sim, g(sim.pos), g(sim.vel), g(sim.mass), sim.cs.cpu().numpy()
+
+
+def _mark(sim, max_mass=4.0):
+    from granular_gpu_amd import _lib
+    from granular_gpu_amd.device import _ptr, _stream
+    _lib.check("gg_merge_mark", sim.lib.gg_merge_mark(
+        C.byref(sim.set), C.byref(sim.ad), _ptr(sim.cs), max_mass, C.byref(sim.ws), _stream()))
+    n = sim.n
+    return (sim.remove[:n].cpu().numpy(), sim.merge[:n].cpu().numpy(), sim.mv[:n].cpu().numpy())
+
+
+def _oracle_mark(s, pos, vel, mass, surf, sd, cs, max_mass=4.0):
+    n = pos.shape[0]
+    rem, mer, mv = np.zeros(n, np.int32), np.zeros(n, np.float32), np.zeros((n, 3), np.float32)
+    po.load().oracle_merge_mark(n, pos.reshape(-1), mass, vel.reshape(-1), surf, sd, rem, mer,
+                                mv.reshape(-1), cs, po.params_from(s, 3, 5), max_mass, None, None)
+    return rem, mer, mv
+
+
+@pytest.mark.parametrize("n,crowd", [(1, 0), (3, 0), (5, 1), (61, 0.5), (700, 0.0), (1500, 0.4),
+                                     (2200, 0.9)])
+def test_stencil_passes_equal_oracle(gpu, n, crowd):
+    from granular_gpu_amd import _lib
+    from granular_gpu_amd.device import _ptr, _stream
+    s = _cloud(n, n, crowd)
+    sim, pos, vel, mass, cs = _sorted_sim(s)
+    p, lib = po.params_from(s, 3, 5), po.load()
+    _lib.check("gg_surface", sim.lib.gg_surface(C.byref(sim.set), _ptr(sim.cs),
+                                                C.byref(sim.params), C.byref(sim.ws), _stream()))
+    _lib.check("gg_surface_distance", sim.lib.gg_surface_distance(
+        C.byref(sim.set), _ptr(sim.cs), C.byref(sim.ws), _stream()))
+    cover, surf, sd = np.zeros((n, 3), np.float32), np.zeros(n, np.int32), np.zeros(n, np.float32)
+    lib.oracle_surface(n, pos.reshape(-1), mass, cs, p, cover.reshape(-1), surf)
+    lib.oracle_surface_distance(n, pos.reshape(-1), surf, cs, p, sd)
+    assert np.array_equal(sim.surface[:n].cpu().numpy(), surf)
+    assert np.array_equal(sim.sd[:n].cpu().numpy(), sd)
+    # marking with every particle deep, so that the crowd takes part
+    surf[:], sd[:] = 0, 1e5
+    sim.surface[:n], sim.sd[:n] = 0, 1e5
+    for a, b in zip(_mark(sim, 16.0), _oracle_mark(s, pos, vel, mass, surf, sd, cs, 16.0)):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("lines,length", [(1, 2), (1, 3000), (3, 1365), (5, 1200)])
+def test_claim_chains_equal_oracle(gpu, lines, length):
+    # (up to 4096 undecided claims are finished on chip, more in memory)
+    s = _lines(lines, length)
+    sim, pos, vel, mass, cs = _sorted_sim(s)
+    n = s.n
+    surf, sd = np.zeros(n, np.int32), np.full(n, 1e5, np.float32)
+    sim.surface[:n], sim.sd[:n] = 0, 1e5
+    want = _oracle_mark(s, pos, vel, mass, surf, sd, cs)
+    assert (want[0] == -1).sum() >= n - 2 * lines
+    for a, b in zip(_mark(sim), want):
+        assert np.array_equal(a, b)
