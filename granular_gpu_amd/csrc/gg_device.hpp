@@ -124,6 +124,39 @@ __device__ __forceinline__ void stencil_rows(int bx, int by, int bz, const DevGr
   }
 }
 
+// The index ranges [a, b) over two cell tables of the nine rows of a stencil,
+// in scan order, each loaded one row ahead of its use: f(a0, b0, a1, b1) is
+// called per row (empty ranges included), so a scan waits for one round of
+// table loads, not for one per row.
+template <class F>
+__device__ __forceinline__ void stencil_rows_ahead(bool ok, int bx, int by, int bz,
+                                                   const DevGrid &g, const int *__restrict__ t0,
+                                                   const int *__restrict__ t1, F &&f) {
+  const int z0 = bz - 1 > 0 ? bz - 1 : 0;
+  const int z1 = bz + 1 < g.cz - 1 ? bz + 1 : g.cz - 1;
+  int n0 = 0, m0 = 0, n1 = 0, m1 = 0;
+  auto load = [&](int r) {
+    n0 = m0 = n1 = m1 = 0;
+    const int x = bx + r / 3 - 1, y = by + r % 3 - 1;
+    if (ok && z0 <= z1 && x >= 0 && x < g.cx && y >= 0 && y < g.cy) {
+      const int c = (x * g.cy + y) * g.cz;
+      n0 = t0[c + z0];
+      m0 = t0[c + z1 + 1];
+      if (t1) {
+        n1 = t1[c + z0];
+        m1 = t1[c + z1 + 1];
+      }
+    }
+  };
+  load(0);
+#pragma unroll 1
+  for (int r = 0; r < 9; ++r) {
+    const int a0 = n0, b0 = m0, a1 = n1, b1 = m1;
+    if (r < 8) load(r + 1);
+    f(a0, b0, a1, b1);
+  }
+}
+
 // Element i of a packed float3 array (x, y, z at 3i), read with one 12-byte
 // load per lane instead of three scalar ones.
 struct Packed3 {
@@ -150,16 +183,16 @@ __device__ __forceinline__ float radius_contact(float m, double denom) {
 
 // Slot of the member v = raw[d] of a cell in a stable sort, and its cell c:
 // the cell's first slot plus the members of a smaller index.  Cells of more
-// than kBigLds members are in order already.  Counting a cell's members
-// costs a load and two instructions each: nothing at the usual 8 a cell, and
-// about 15 us at 4096 (the sentinel cell of particles that left the grid),
-// which two launches for a sort of larger cells cost every build.
+// than limit members are in order already.  Counting a cell's members costs a
+// load and two instructions each: nothing at the usual 8 a cell, about 10 us
+// at 1024 (a sentinel cell of particles that left the grid), where sorting
+// the larger cells took two launches of every build.
 __device__ __forceinline__ int sorted_slot(const int *__restrict__ raw, const int *__restrict__ key,
-                                           const int *__restrict__ cell_start, int d, int v,
-                                           int &c) {
+                                           const int *__restrict__ cell_start, int limit, int d,
+                                           int v, int &c) {
   c = key[v];
   const int s = cell_start[c], e = cell_start[c + 1];
-  if (e - s > kBigLds) return d;
+  if (e - s > limit) return d;
   int rank = 0, k = s;
   for (; k + 8 <= e; k += 8) {
     int r[8];

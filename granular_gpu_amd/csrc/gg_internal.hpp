@@ -11,12 +11,18 @@
 namespace gg {
 
 constexpr int kBlock = 256;        // threads per block for particle kernels
-constexpr int kScanTile = 2048;    // elements per block in the cell-table scan
+constexpr int kScanTile = 2048;    // elements per block in the cell-table scan (4 times that
+                                   // for tables of more than kScanWide tiles)
+constexpr int kScanWide = 256;
 constexpr int kScanMaxParts = 8192;
-constexpr int kBigLds = 4096;      // cells up to this size are ranked one thread per entry
-constexpr int kHugeChunks = 256;   // blocks compacting each larger cell
+// Cells up to big_cell(n) members are ranked one thread per entry, larger ones
+// compacted by kHugeChunks blocks.  A set that cannot hold a cell of more than
+// kBigSet needs no launches for the latter.
+constexpr int kBigCell = 1024, kBigSet = 4096;
+__host__ __device__ inline int big_cell(int n) { return n <= kBigSet ? kBigSet : kBigCell; }
+constexpr int kHugeChunks = 256;
 constexpr int kScanSync = 8;       // ctr2[8..9]: the scan's tile and finish counters
-constexpr int kHugeCounter = 63;   // ctr[63]: cells larger than kBigLds in this build
+constexpr int kHugeCounter = 63;   // ctr[63]: cells larger than big_cell(n) in this build
 constexpr double kPiD = 3.14159265358979323846;
 constexpr float kPiF = 3.14159265358979323846f;
 // A particle's list stays exact while its own accumulated correction and
@@ -62,7 +68,7 @@ struct Layout {
   size_t perm;     // int[cmax]      sorted slot -> old index
   size_t itmp;     // int[cmax]      cell order as scattered (before the stable ranking)
   size_t part;     // int[parts+1]   scan tile states, zero between scans
-  size_t big;      // int[C+1]       record of each cell of more than kBigLds members
+  size_t big;      // int[C+1]       record of each cell of more than big_cell(n) members
   size_t ctr;      // int[64]        device counters
   size_t ctr2;     // int[64]        adaptive and scan counters
   size_t dirty;    // int[C+1]       cells near a particle past half the skin

@@ -80,40 +80,53 @@ __device__ __forceinline__ void tile_store(unsigned int *p, unsigned int v) {
 // order the blocks start (sync[0]), so a tile only waits for tiles whose
 // blocks already run and publish their sums without waiting: every wait ends.
 // The last block to finish (sync[1]) leaves states and counters zero for the
-// next launch.  huge (optional): cells of more than kBigLds entries are
-// recorded as {cell, INT_MAX, 0} and found again through at_huge[cell].
+// next launch.  huge (optional): cells of more than `limit` entries are
+// recorded, found again through at_huge[cell], their chunk words cleared.
+// SUB: sub-tiles of kScanTile elements per tile (fewer tiles to order and to
+// look back over in a long table: 1.6M cells 30 -> 21 us).
+template <int SUB>
 __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
                                                  unsigned int *__restrict__ state,
                                                  int *__restrict__ sync, int *__restrict__ out,
                                                  int *__restrict__ huge, int *__restrict__ at_huge,
-                                                 int *__restrict__ nhuge) {
+                                                 int *__restrict__ hcnt, int *__restrict__ nhuge,
+                                                 int limit) {
   __shared__ int tile_s, excl_s;
-  __shared__ int wtot[kBlock / 64];
+  __shared__ int wtot[SUB][kBlock / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const bool alone = gridDim.x == 1;  // one tile: nothing to exchange
   if (!alone && threadIdx.x == 0) tile_s = atomicAdd(&sync[0], 1);
   __syncthreads();
   const int tile = alone ? 0 : tile_s;
-  const int base = tile * kScanTile + threadIdx.x * 8;
-  int loc[8];
-  int s = 0;
+  const int base = tile * (SUB * kScanTile) + threadIdx.x * 8;
+  int loc[SUB][8], s[SUB], inc[SUB];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    loc[k] = base + k < m ? in[base + k] : 0;
-    s += loc[k];
+  for (int q = 0; q < SUB; ++q) {
+    s[q] = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int idx = base + q * kScanTile + k;
+      loc[q][k] = idx < m ? in[idx] : 0;
+      s[q] += loc[q][k];
+    }
   }
-  int inc = s;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
+#pragma unroll
+  for (int q = 0; q < SUB; ++q) {
+    inc[q] = s[q];
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(inc[q], o, 64);
+      if (lane >= o) inc[q] += v;
+    }
+    if (lane == 63) wtot[q][wid] = inc[q];
   }
-  if (lane == 63) wtot[wid] = inc;
   __syncthreads();
-  int woff = 0, total = 0;
-  for (int w = 0; w < kBlock / 64; ++w) {
-    if (w < wid) woff += wtot[w];
-    total += wtot[w];
-  }
+  int total = 0, woff[SUB];
+#pragma unroll
+  for (int q = 0; q < SUB; ++q)
+    for (int w = 0; w < kBlock / 64; ++w) {
+      if (w == wid) woff[q] = total;
+      total += wtot[q][w];
+    }
   if (alone) {
     if (threadIdx.x == 0) excl_s = 0;
   } else if (wid == 0) {
@@ -139,23 +152,25 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
     }
   }
   __syncthreads();
-  int run = excl_s + woff + inc - s;
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = base + k;
-    if (idx < m) {
-      out[idx] = run;
-      in[idx] = 0;
-      if (idx == m - 1) out[m] = run + loc[k];
-      if (huge && loc[k] > kBigLds) {
-        const int h = atomicAdd(nhuge, 1);
-        huge[3 * h] = idx;
-        huge[3 * h + 1] = 0x7fffffff;
-        huge[3 * h + 2] = 0;
-        at_huge[idx] = h;
+  for (int q = 0; q < SUB; ++q) {
+    int run = excl_s + woff[q] + inc[q] - s[q];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int idx = base + q * kScanTile + k;
+      if (idx < m) {
+        out[idx] = run;
+        in[idx] = 0;
+        if (idx == m - 1) out[m] = run + loc[q][k];
+        if (huge && loc[q][k] > limit) {
+          const int h = atomicAdd(nhuge, 1);
+          huge[h] = idx;
+          at_huge[idx] = h;
+          for (int p = 0; p < kHugeChunks; ++p) hcnt[h * kHugeChunks + p] = 0;
+        }
       }
+      run += loc[q][k];
     }
-    run += loc[k];
   }
   if (!alone && wid == 0) {
     // every block has read the states it needs before it counts itself
@@ -168,13 +183,25 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
   }
 }
 
-// raw[cell_start + arrival slot] = i; for the cells recorded as huge also the
-// range [lo, hi) of their members' indices.
+// Chunk p of kHugeChunks equal parts of [0, n), and the chunk of index i.
+__device__ __forceinline__ void huge_chunk(int n, int p, int &a, int &b) {
+  a = (int)((long long)n * p / kHugeChunks);
+  b = (int)((long long)n * (p + 1) / kHugeChunks);
+}
+__device__ __forceinline__ int chunk_of(int i, int n) {
+  return (int)((((long long)i + 1) * kHugeChunks - 1) / n);
+}
+
+// raw[cell_start + arrival slot] = i; for the cells recorded as huge also a
+// mark on each chunk of indices that holds members (plain stores of the same
+// value: atomics on a cell's range took 140 us with 640k particles in 64
+// sentinel cells).
 __global__ void __launch_bounds__(kBlock) k_scatter(const int *__restrict__ key,
                                                     const int *__restrict__ slot, int n,
                                                     const int *__restrict__ cell_start,
-                                                    int *__restrict__ raw, int *__restrict__ huge,
-                                                    const int *__restrict__ at_huge) {
+                                                    int *__restrict__ raw,
+                                                    const int *__restrict__ at_huge,
+                                                    int *__restrict__ hcnt, int limit) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   int h = -1;
   if (i < n) {
@@ -182,17 +209,18 @@ __global__ void __launch_bounds__(kBlock) k_scatter(const int *__restrict__ key,
     const int s = cell_start[c];
     const int d = s + slot[i];
     if (d >= 0 && d < n) raw[d] = i;
-    if (huge && cell_start[c + 1] - s > kBigLds) h = at_huge[c];
+    if (hcnt && cell_start[c + 1] - s > limit) h = at_huge[c];
   }
-  // one pair of atomics per wave and huge cell (lanes are in index order)
+  // each wave's first and last member of a cell mark their chunks and those
+  // between
   const int lane = threadIdx.x & 63;
   unsigned long long m = __ballot(h >= 0);
   while (m) {
     const int first = __ffsll((long long)m) - 1;
     const unsigned long long mine = __ballot(h == __shfl(h, first, 64));
     if (lane == first) {
-      atomicMin(&huge[3 * h + 1], i);
-      atomicMax(&huge[3 * h + 2], i + 64 - __clzll((long long)mine) - lane);
+      const int last = chunk_of(i + 63 - __clzll((long long)mine) - lane, n);
+      for (int p = chunk_of(i, n); p <= last; ++p) hcnt[h * kHugeChunks + p] = 1;
     }
     m &= ~mine;
   }
@@ -207,7 +235,7 @@ __global__ void __launch_bounds__(kBlock) k_rank(const int *__restrict__ raw, in
   if (d >= n) return;
   int c;
   const int v = raw[d];
-  perm[sorted_slot(raw, key, cell_start, d, v, c)] = v;
+  perm[sorted_slot(raw, key, cell_start, big_cell(n), d, v, c)] = v;
 }
 
 // A set's payload permuted into the staging arrays (and back, in place, by
@@ -232,7 +260,7 @@ __global__ void __launch_bounds__(kBlock)
   for (int k = 0; k < 5; ++k)
     if (src.w[k]) w[k] = src.w[k][v];
   int c;
-  const int o = sorted_slot(raw, key, cell_start, d, v, c);
+  const int o = sorted_slot(raw, key, cell_start, big_cell(n), d, v, c);
   tmp.pos[o] = x;
   if (src.vel) tmp.vel[o] = u;
 #pragma unroll
@@ -252,29 +280,24 @@ __global__ void __launch_bounds__(kBlock) k_payload_back(int n, Payload dst, Pay
     if (dst.w[k]) dst.w[k][i] = tmp.w[k][i];
 }
 
-// Chunk p of kHugeChunks equal parts of [lo, hi).
-__device__ __forceinline__ void huge_chunk(int lo, int hi, int p, int &a, int &b) {
-  const long long w = (long long)hi - lo;
-  a = lo + (int)(w * p / kHugeChunks);
-  b = lo + (int)(w * (p + 1) / kHugeChunks);
-}
-
 // Block p counts the members of each recorded cell in its chunk of the
-// cell's range: cnt[h * kHugeChunks + p].
-__global__ void __launch_bounds__(kBlock) k_huge_count(const int *__restrict__ key,
+// indices, where it is marked: cnt[h * kHugeChunks + p].
+__global__ void __launch_bounds__(kBlock) k_huge_count(const int *__restrict__ key, int n,
                                                        const int *__restrict__ ctr,
                                                        const int *__restrict__ huge,
                                                        int *__restrict__ cnt) {
   __shared__ int red[kBlock / 64];
   const int nh = ctr[kHugeCounter];
   const int p = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int a = 0, b = 0;
+  huge_chunk(n, p, a, b);
   for (int h = 0; h < nh; ++h) {
-    const int c = huge[3 * h];
-    int a = 0, b = 0;
-    huge_chunk(huge[3 * h + 1], huge[3 * h + 2], p, a, b);
+    if (cnt[h * kHugeChunks + p] == 0) continue;  // (the same for the whole block)
+    const int c = huge[h];
     int m = 0;
     for (int i = a + threadIdx.x; i < b; i += blockDim.x) m += key[i] == c ? 1 : 0;
-    for (int o = 32; o > 0; o >>= 1) m += __shfl_xor(m, o, 64);
+    m = wave_sum(m);
+    __syncthreads();
     if (lane == 0) red[wid] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -282,14 +305,13 @@ __global__ void __launch_bounds__(kBlock) k_huge_count(const int *__restrict__ k
       for (int w = 0; w < kBlock / 64; ++w) t += red[w];
       cnt[h * kHugeChunks + p] = t;
     }
-    __syncthreads();
   }
 }
 
 // Block p writes the members of each recorded cell found in its chunk, in
 // index order, after those of the chunks before it: a stable compaction of
-// {i in [lo, hi) : key[i] == c} into the cell's slots.
-__global__ void __launch_bounds__(kBlock) k_huge_write(const int *__restrict__ key,
+// {i : key[i] == c} into the cell's slots.
+__global__ void __launch_bounds__(kBlock) k_huge_write(const int *__restrict__ key, int n,
                                                        const int *__restrict__ cell_start,
                                                        const int *__restrict__ ctr,
                                                        const int *__restrict__ huge,
@@ -298,15 +320,17 @@ __global__ void __launch_bounds__(kBlock) k_huge_write(const int *__restrict__ k
   __shared__ int wcnt[kBlock / 64];
   const int nh = ctr[kHugeCounter];
   const int p = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int a = 0, b = 0;
+  huge_chunk(n, p, a, b);
   for (int h = 0; h < nh; ++h) {
-    const int c = huge[3 * h];
+    if (cnt[h * kHugeChunks + p] == 0) continue;
+    const int c = huge[h];
     const int s = cell_start[c], len = cell_start[c + 1] - s;
-    int a = 0, b = 0;
-    huge_chunk(huge[3 * h + 1], huge[3 * h + 2], p, a, b);
     // members in the chunks before this one
     int before = 0;
     for (int q = threadIdx.x; q < p; q += blockDim.x) before += cnt[h * kHugeChunks + q];
-    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    before = wave_sum(before);
+    __syncthreads();
     if (lane == 0) wcnt[wid] = before;
     __syncthreads();
     int base = 0;
@@ -369,19 +393,25 @@ __global__ void __launch_bounds__(kBlock) k_pack_boundary(const float *__restric
 static inline int blocks_for(long long n) { return (int)((n + kBlock - 1) / kBlock); }
 
 static int launch_scan(int *in, int m, int *out, const gg_workspace *ws, int *huge, int *at_huge,
-                       int *nhuge, hipStream_t st) {
+                       int *hcnt, int *nhuge, int limit, hipStream_t st) {
   Layout L = make_layout(ws->capacity, ws->boundary_capacity, ws->grid, ws->max_sweeps, ws->gmax,
                          ws->bmax);
   const int np = (m + kScanTile - 1) / kScanTile;
-  k_scan<<<np, kBlock, 0, st>>>(in, m, at<unsigned int>(ws, L.part),
-                                at<int>(ws, L.ctr2) + kScanSync, out, huge, at_huge, nhuge);
+  unsigned int *state = at<unsigned int>(ws, L.part);
+  int *sync = at<int>(ws, L.ctr2) + kScanSync;
+  if (np <= kScanWide)
+    k_scan<1><<<np, kBlock, 0, st>>>(in, m, state, sync, out, huge, at_huge, hcnt,
+                                      nhuge, limit);
+  else
+    k_scan<4><<<(np + 3) / 4, kBlock, 0, st>>>(in, m, state, sync, out, huge, at_huge, hcnt,
+                                      nhuge, limit);
   GG_LAUNCH_CHECK();
   return GG_OK;
 }
 
 // Hash (or the given keys), counting sort and cell table for n particles:
 // the workspace's itmp array ends with each cell's members (ascending in
-// cells of more than kBigLds, in any order below that: sorted_slot ranks
+// cells of more than big_cell(n), in any order below that: sorted_slot ranks
 // them where they are consumed).
 int sort_by_cell_keys(const float *pos, const int *keys_in, int n, int *cell_start,
                       const gg_workspace *ws, hipStream_t st, int *key_copy) {
@@ -396,22 +426,24 @@ int sort_by_cell_keys(const float *pos, const int *keys_in, int n, int *cell_sta
   int *at_huge = at<int>(ws, L.big);
   int *ctr = at<int>(ws, L.ctr);
   // the huge-cell records and per-chunk counts live in the permutation's
-  // array, which is written after the sort: (3 + kHugeChunks) ints per cell
-  // of more than kBigLds particles (at most n / kBigLds of them)
-  int *huge = n > kBigLds ? at<int>(ws, L.perm) : nullptr;
-  int *hcnt = at<int>(ws, L.perm) + 3 * (n / kBigLds + 1);
+  // array, which is written after the sort: (1 + kHugeChunks) ints per cell
+  // of more than kBigCell particles (at most n / kBigCell of them)
+  const int limit = big_cell(n);
+  int *huge = n > limit ? at<int>(ws, L.perm) : nullptr;
+  int *hcnt = huge ? huge + n / kBigCell + 1 : nullptr;
   const int nb = n > 0 ? blocks_for(n) : 1;
   k_hash_count<<<nb, kBlock, 0, st>>>(pos, keys_in, n, g, key, slot, count, ctr, key_copy);
   GG_LAUNCH_CHECK();
-  GG_TRY(launch_scan(count, m, cell_start, ws, huge, at_huge, ctr + kHugeCounter, st));
+  GG_TRY(launch_scan(count, m, cell_start, ws, huge, at_huge, hcnt, ctr + kHugeCounter, limit,
+                     st));
   if (n > 0) {
-    k_scatter<<<nb, kBlock, 0, st>>>(key, slot, n, cell_start, raw, huge, at_huge);
+    k_scatter<<<nb, kBlock, 0, st>>>(key, slot, n, cell_start, raw, at_huge, hcnt, limit);
     GG_LAUNCH_CHECK();
   }
   if (huge) {
-    k_huge_count<<<kHugeChunks, kBlock, 0, st>>>(key, ctr, huge, hcnt);
+    k_huge_count<<<kHugeChunks, kBlock, 0, st>>>(key, n, ctr, huge, hcnt);
     GG_LAUNCH_CHECK();
-    k_huge_write<<<kHugeChunks, kBlock, 0, st>>>(key, cell_start, ctr, huge, hcnt, raw);
+    k_huge_write<<<kHugeChunks, kBlock, 0, st>>>(key, n, cell_start, ctr, huge, hcnt, raw);
     GG_LAUNCH_CHECK();
   }
   return GG_OK;
@@ -438,7 +470,7 @@ int sort_permutation(int n, const int *cell_start, const gg_workspace *ws, hipSt
 int scan_exclusive(int *in, int m, int *out, const gg_workspace *ws, hipStream_t st) {
   if (m <= 0) return GG_OK;
   if ((long long)m > (long long)kScanTile * kScanMaxParts) return GG_ERR_CAPACITY;
-  return launch_scan(in, m, out, ws, nullptr, nullptr, nullptr, st);
+  return launch_scan(in, m, out, ws, nullptr, nullptr, nullptr, nullptr, 0, st);
 }
 
 int gather_inplace(void *arr, int words, const int *perm, int n, void *tmp, hipStream_t st) {

@@ -424,20 +424,28 @@ __global__ void __launch_bounds__(256)
   const float qz = pos[3 * i + 2] + radius * templ(k, 2);
   float best = INFINITY;
   int bj = -1;
-  int bx, by, bz;
-  if (floor_cell(qx, qy, qz, fg, bx, by, bz)) {
-    stencil_rows(bx, by, bz, fg, fcs, [&](int j0, int j1) {
-      for (int j = j0; j < j1; ++j) {
-        const Packed3 f = ld3(fpos, j);
-        const float dx = f.x - qx, dy = f.y - qy, dz = f.z - qz;
+  // eight candidates' loads in flight (one after another, a chain of 216,
+  // 64k coarse particles took 126 us; now 94)
+  int bx = 0, by = 0, bz = 0;
+  const bool ok = floor_cell(qx, qy, qz, fg, bx, by, bz);
+  stencil_rows_ahead(ok, bx, by, bz, fg, fcs, nullptr, [&](int j0, int j1, int, int) {
+    for (int j = j0; j < j1; j += 8) {
+      Packed3 f[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) f[u] = ld3(fpos, j + u < j1 ? j + u : j);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float dx = f[u].x - qx, dy = f[u].y - qy, dz = f[u].z - qz;
         const float dd = dx * dx + dy * dy + dz * dz;
-        if (dd < best || (dd == best && j < bj)) {
+        // (indices ascend, so the first of equals is the lowest; a slot past
+        // the row repeats its first candidate and is never smaller)
+        if (dd < best) {
           best = dd;
-          bj = j;
+          bj = j + u < j1 ? j + u : j;
         }
       }
-    });
-  }
+    }
+  });
   const size_t o = (size_t)i * kOut + 3 * k;
   if (bj < 0) {
     y[o] = y[o + 1] = y[o + 2] = 0.0f;
@@ -1378,6 +1386,7 @@ struct SideStream {
   hipStream_t st = nullptr;
   hipEvent_t fork = nullptr, join = nullptr, flags = nullptr;
 };
+constexpr int kFlagsFirst = 262144;
 static int side_stream(SideStream *&out) {
   static std::mutex mu;
   static SideStream per_dev[64];
@@ -1437,19 +1446,31 @@ extern "C" int gg_upsample_mlp(const gg_particles *coarse, const int *cs,
   // template), beside the features pass and the network on the caller's
   // stream (disjoint outputs); the network waits for the flags only.  Fused
   // into the features pass instead, the fallback would start only after it.
+  // Up to kFlagsFirst particles the flags come first on the caller's stream
+  // instead: a wait between streams costs more than the overlap gives (27k
+  // 68.6 -> 62.0 us a call, 92k 82.1 -> 79.4, 216k 96.3 -> 94.2; at 332k
+  // side by side is ahead, 116.8 against 121.9, at 512k 150.8 against 159.7).
   SideStream *side = nullptr;
   GG_TRY(side_stream(side));
-  if (hipEventRecord(side->fork, stream) != hipSuccess ||
-      hipStreamWaitEvent(side->st, side->fork, 0) != hipSuccess)
-    return GG_ERR_HIP;
-  prof_begin(GG_STAGE_MLP_FALLBACK, side->st);
-  k_zero_int<<<1, 1, 0, side->st>>>(fb_count);
-  k_mlp_flags<<<nblocks(n, 256), 256, 0, side->st>>>(
+  const bool first = n <= kFlagsFirst;
+  auto fork = [&]() {
+    return hipEventRecord(side->fork, stream) == hipSuccess &&
+           hipStreamWaitEvent(side->st, side->fork, 0) == hipSuccess;
+  };
+  if (!first && !fork()) return GG_ERR_HIP;
+  const hipStream_t fs = first ? stream : side->st;
+  prof_begin(GG_STAGE_MLP_FALLBACK, fs);
+  k_zero_int<<<1, 1, 0, fs>>>(fb_count);
+  k_mlp_flags<<<nblocks(n, 256), 256, 0, fs>>>(
       n, pos, reinterpret_cast<const float *>(boundary->pos), bcs, g, mlp_const(c), flags,
       fb_list, fb_count);
-  if (fallback_count) k_copy_int<<<1, 1, 0, side->st>>>(fb_count, fallback_count);
-  const bool flags_ok =
-      hipGetLastError() == hipSuccess && hipEventRecord(side->flags, side->st) == hipSuccess;
+  if (fallback_count) k_copy_int<<<1, 1, 0, fs>>>(fb_count, fallback_count);
+  bool flags_ok = hipGetLastError() == hipSuccess;
+  if (first) {
+    if (!flags_ok || !fork()) return GG_ERR_HIP;
+  } else {
+    flags_ok = flags_ok && hipEventRecord(side->flags, side->st) == hipSuccess;
+  }
   if (flags_ok)
     k_mlp_fallback<<<cus * 8, 256, 0, side->st>>>(
         fb_list, fb_count, pos, vel, cs, reinterpret_cast<const float *>(boundary->pos), bcs,
@@ -1471,7 +1492,8 @@ extern "C" int gg_upsample_mlp(const gg_particles *coarse, const int *cs,
     k_mlp_features<1, 16><<<nblocks(n, 256), 256, 0, stream>>>(n, pos, vel, cs, g,
                                                                mlp_const(c), feat, nullptr);
   if (hipGetLastError() != hipSuccess) frc = GG_ERR_HIP;
-  if (frc == GG_OK && hipStreamWaitEvent(stream, side->flags, 0) != hipSuccess) frc = GG_ERR_HIP;
+  if (frc == GG_OK && !first && hipStreamWaitEvent(stream, side->flags, 0) != hipSuccess)
+    frc = GG_ERR_HIP;
   if (frc != GG_OK) {
     (void)hipStreamWaitEvent(stream, side->join, 0);
     return frc;

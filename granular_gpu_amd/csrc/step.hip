@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(kBlock)
     const float r = radius_contact(m, denom);
     // o's place in the stable order (identity without a sort)
     int i = d, c = 0;
-    if (raw) i = sorted_slot(raw, key, cell_start, d, o, c);
+    if (raw) i = sorted_slot(raw, key, cell_start, big_cell(n), d, o, c);
     x0[i] = make_float4(px, py, pz, r);
     off0[i] = make_float4(Dx, Dy, Dz, 0.0f);
     d0[i] = make_float4(Dx, Dy, Dz, 0.0f);
@@ -350,7 +350,7 @@ __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
 // time): lanes 0..8 of a group read the nine rows' ranges at once, the group
 // tests 16 candidates of a row at a time, three rows' loads in flight, and a
 // ballot gives each hit its place in the list.  Twice the instructions of
-// k_nlist per particle, so not for larger sets.  @WIDE
+// k_nlist per particle, so not for larger sets.
 constexpr int kWideListMax = 65536;
 template <bool SCENES>
 __global__ void __launch_bounds__(64) k_nlist_wide(ListArgs a) {
