@@ -173,7 +173,10 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
     }
   }
   if (!alone && wid == 0) {
-    // every block has read the states it needs before it counts itself
+    // A block counts itself when it has read the states it needs and its own
+    // stores to them have been performed: the states go through to memory, so
+    // an empty store counter means that, and none can land after the zeros.
+    __builtin_amdgcn_s_waitcnt(0);
     int done = 0;
     if (lane == 0) done = atomicAdd(&sync[1], 1);
     if (__shfl(done, 0, 64) == (int)gridDim.x - 1) {
