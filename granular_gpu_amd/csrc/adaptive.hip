@@ -113,7 +113,7 @@ __device__ __forceinline__ void group_scan(const Group &G, const float *__restri
           v[u] = a[j];
         }
       }
-      __builtin_amdgcn_wave_barrier();
+      converge();
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int j = c + 16 * u + G.sub;
@@ -137,9 +137,7 @@ struct Hits {
   __device__ __forceinline__ void add(const Group &G, bool hit, int j) {
     const unsigned int m = group_ballot(G, hit);
     if (hit) list[count + __popc(m & ((1u << G.sub) - 1u))] = j;
-    // (lanes that skip the store wait here: a lane running ahead into the
-    // next turn of a loop would be missing from this ballot)
-    __builtin_amdgcn_wave_barrier();
+    converge();
     count += __popc(m);
   }
 };
@@ -197,7 +195,7 @@ __global__ void __launch_bounds__(64)
         const Packed3 q = ld3(pos, H.list[t + G.sub]);
         u = nrm(x.x - q.x, x.y - q.y, x.z - q.z);
       }
-      __builtin_amdgcn_wave_barrier();
+      converge();
       cx = add_row(cx, u.x);
       cy = add_row(cy, u.y);
       cz = add_row(cz, u.z);
@@ -231,7 +229,7 @@ __global__ void __launch_bounds__(64)
         const float3 u = nrm(q.x - x.x, q.y - x.y, q.z - x.z);
         if (u.x * cv.x + u.y * cv.y + u.z * cv.z >= 0.5f) vote = true;
       }
-      __builtin_amdgcn_wave_barrier();
+      converge();
     }
   };
   if (partial) {
@@ -354,7 +352,7 @@ __global__ void __launch_bounds__(64)
           }
         }
       }
-      __builtin_amdgcn_wave_barrier();
+      converge();
       ld = add_row(ld, m);
     }
   };

@@ -11,6 +11,11 @@
 
 namespace gg {
 
+// The wave's lanes meet here: without it the compiler may let the lanes that
+// skip a conditional store run ahead into the next turn of a loop around it,
+// and a ballot there sees some of the lanes only (it did).
+__device__ __forceinline__ void converge() { __builtin_amdgcn_wave_barrier(); }
+
 struct DevGrid {
   float L, invL;  // cell length and the rounded 1 / L
   int cx, cy, cz;

@@ -140,6 +140,7 @@ __global__ void __launch_bounds__(kBlock) k_scan(int *__restrict__ in, int m,
       while (__any(v == 0u)) {
         __builtin_amdgcn_s_sleep(1);
         if (v == 0u) v = tile_load(&state[t]);
+        converge();
       }
       const unsigned long long pre = __ballot((v & kTilePrefix) != 0u);
       const int upto = pre ? __ffsll((long long)pre) - 1 : 63;
@@ -225,6 +226,7 @@ __global__ void __launch_bounds__(kBlock) k_scatter(const int *__restrict__ key,
       const int last = chunk_of(i + 63 - __clzll((long long)mine) - lane, n);
       for (int p = chunk_of(i, n); p <= last; ++p) hcnt[h * kHugeChunks + p] = 1;
     }
+    converge();
     m &= ~mine;
   }
 }

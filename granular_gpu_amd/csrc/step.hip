@@ -36,11 +36,6 @@
 
 namespace gg {
 
-// The wave's lanes meet here: without it the compiler may let the lanes that
-// skip a conditional store run ahead into the next turn of a loop around it,
-// and a ballot there sees some of the lanes only (it did).
-__device__ __forceinline__ void converge() { __builtin_amdgcn_wave_barrier(); }
-
 // Positions for the list build's prefilter in 8 bytes: x, y, z in units of
 // L / 4096 modulo 2^16 (16 cells: differences inside a stencil are exact),
 // and minus the radius in units, rounded up, at most 4 cells.  Rounding moves
@@ -819,6 +814,7 @@ __device__ __forceinline__ void scan_by_wave(const SweepArgs &a, int iq) {
                          nqb, nqg);
   if ((threadIdx.x & 63) == 0)
     sweep_store<LAST_STAB>(a, iq, bq, oq, qb, qg, nqb + nqg, a.meta[iq].w, lq);
+  converge();  // (callers go on to the next particle)
 }
 
 // One sweep.  What bounds it at size is the gathers: two 16-byte loads per
