@@ -1405,29 +1405,37 @@ static int launch_infer(int n, const uint2 *feat4, const int *flags, const float
 }
 
 // A second stream per device (default priority) on which the teacher
-// fallback runs beside the network kernel, with the two events that fork it
+// fallback runs beside the network kernel, with the events that fork it
 // from and join it back into the caller's stream.  Created on first use,
-// kept for the life of the process.
+// kept for the life of the process.  A call holds the lock from its first
+// use of an event to its last: between one caller's record and its wait,
+// another's record would make it wait for the wrong stream, and the fallback
+// read a list that is not written yet.
 struct SideStream {
+  std::mutex mu;
   hipStream_t st = nullptr;
   hipEvent_t fork = nullptr, join = nullptr, flags = nullptr;
 };
 constexpr int kFlagsFirst = 262144;
 static int side_stream(SideStream *&out) {
-  static std::mutex mu;
   static SideStream per_dev[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return GG_ERR_HIP;
-  std::lock_guard<std::mutex> lock(mu);
-  SideStream &s = per_dev[dev];
-  if (!s.st) {
-    if (hipStreamCreateWithFlags(&s.st, hipStreamNonBlocking) != hipSuccess) return GG_ERR_HIP;
-    if (hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s.flags, hipEventDisableTiming) != hipSuccess)
-      return GG_ERR_HIP;
+  out = &per_dev[dev];
+  return GG_OK;
+}
+// (with the side stream's lock held)
+static int make_side_stream(SideStream &s) {
+  if (s.st) return GG_OK;
+  hipStream_t st = nullptr;
+  if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return GG_ERR_HIP;
+  if (hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&s.flags, hipEventDisableTiming) != hipSuccess) {
+    (void)hipStreamDestroy(st);
+    return GG_ERR_HIP;
   }
-  out = &s;
+  s.st = st;
   return GG_OK;
 }
 
@@ -1478,6 +1486,8 @@ extern "C" int gg_upsample_mlp(const gg_particles *coarse, const int *cs,
   // side by side is ahead, 116.8 against 121.9, at 512k 150.8 against 159.7).
   SideStream *side = nullptr;
   GG_TRY(side_stream(side));
+  std::lock_guard<std::mutex> lock(side->mu);
+  GG_TRY(make_side_stream(*side));
   const bool first = n <= kFlagsFirst;
   auto fork = [&]() {
     return hipEventRecord(side->fork, stream) == hipSuccess &&
