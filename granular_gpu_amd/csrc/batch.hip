@@ -29,6 +29,7 @@ struct gg_batch {
   std::vector<hipEvent_t> ev;  // [0] fork, [1 + b] join of branch b
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  bool launched = false;  // exec has been launched since the device was last waited for
 };
 
 namespace gg {
@@ -36,9 +37,18 @@ namespace {
 
 bool block_valid(int b) { return b == 0 || b == 64 || b == 128 || b == 256 || b == 512; }
 
+int launch(gg_batch *b, hipStream_t st) {
+  b->launched = true;
+  return hip_status(hipGraphLaunch(b->exec, st));
+}
+
+// (a graph that could not be waited for is kept for good)
 void release_graph(gg_batch *b) {
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
+  if (!b->launched || wait_for_device()) {
+    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+  }
+  b->launched = false;
   b->exec = nullptr;
   b->graph = nullptr;
 }
@@ -211,7 +221,7 @@ extern "C" int gg_batch_create(const gg_batch_scene *scenes, int nscenes,
 
 extern "C" int gg_batch_step(gg_batch *b, hipStream_t stream) {
   if (!b || !b->exec) return GG_ERR_INVALID;
-  return hip_status(hipGraphLaunch(b->exec, stream));
+  return launch(b, stream);
 }
 
 extern "C" int gg_batch_step_eager(gg_batch *b, hipStream_t stream) {
@@ -269,10 +279,10 @@ extern "C" int gg_batch_autotune(gg_batch *b, int trials, hipStream_t stream,
         c.nlist_block = nl;
         b->cfg = c;
         rc = build_graph(b);
-        if (rc == GG_OK) rc = hip_status(hipGraphLaunch(b->exec, stream));  // warm-up
+        if (rc == GG_OK) rc = launch(b, stream);  // warm-up
         if (rc == GG_OK) rc = hip_status(hipEventRecord(t0, stream));
         for (int t = 0; t < trials && rc == GG_OK; ++t)
-          rc = hip_status(hipGraphLaunch(b->exec, stream));
+          rc = launch(b, stream);
         if (rc == GG_OK) rc = hip_status(hipEventRecord(t1, stream));
         if (rc == GG_OK) rc = hip_status(hipEventSynchronize(t1));
         float ms = 0.0f;

@@ -203,6 +203,17 @@ inline int check_ws(const gg_workspace *ws) {
 
 inline int hip_status(hipError_t e) { return e == hipSuccess ? GG_OK : GG_ERR_HIP; }
 
+// Waits for everything launched on the device, also where another stream of
+// the process is being captured: before a graph with launches in flight is
+// released, whose host objects the runtime's threads may still be using.
+inline bool wait_for_device() {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
+  const bool ok = hipDeviceSynchronize() == hipSuccess;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return ok;
+}
+
 }  // namespace gg
 
 #define GG_LAUNCH_CHECK()                                  \

@@ -91,13 +91,23 @@ struct gg_scenes_graph {
   hipStream_t cap = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  bool launched = false;  // exec has been launched since the device was last waited for
 };
 
 namespace {
 
+int launch(gg_scenes_graph *g, hipStream_t st) {
+  g->launched = true;
+  return hip_status(hipGraphLaunch(g->exec, st));
+}
+
+// (a graph that could not be waited for is kept for good)
 void release(gg_scenes_graph *g) {
-  if (g->exec) (void)hipGraphExecDestroy(g->exec);
-  if (g->graph) (void)hipGraphDestroy(g->graph);
+  if (!g->launched || wait_for_device()) {
+    if (g->exec) (void)hipGraphExecDestroy(g->exec);
+    if (g->graph) (void)hipGraphDestroy(g->graph);
+  }
+  g->launched = false;
   g->exec = nullptr;
   g->graph = nullptr;
 }
@@ -159,7 +169,7 @@ extern "C" int gg_scenes_graph_create(gg_particles *set, int *cell_start,
 
 extern "C" int gg_scenes_graph_launch(gg_scenes_graph *g, hipStream_t stream) {
   if (!g || !g->exec) return GG_ERR_INVALID;
-  return hip_status(hipGraphLaunch(g->exec, stream));
+  return launch(g, stream);
 }
 
 extern "C" int gg_scenes_graph_autotune(gg_scenes_graph *g, int trials, hipStream_t stream,
@@ -201,10 +211,10 @@ extern "C" int gg_scenes_graph_autotune(gg_scenes_graph *g, int trials, hipStrea
       g->params.sweep_block = sw;
       g->params.nlist_block = nl;
       rc = capture(g);
-      if (rc == GG_OK) rc = hip_status(hipGraphLaunch(g->exec, stream));  // warm-up
+      if (rc == GG_OK) rc = launch(g, stream);  // warm-up
       if (rc == GG_OK) rc = hip_status(hipEventRecord(t0, stream));
       for (int t = 0; t < trials && rc == GG_OK; ++t)
-        rc = hip_status(hipGraphLaunch(g->exec, stream));
+        rc = launch(g, stream);
       if (rc == GG_OK) rc = hip_status(hipEventRecord(t1, stream));
       if (rc == GG_OK) rc = hip_status(hipEventSynchronize(t1));
       float ms = 0.0f;

@@ -540,6 +540,7 @@ int gg_scenes_graph_launch(gg_scenes_graph *g, hipStream_t stream);
  * with the fastest; best_ms (optional) = its time per launch. */
 int gg_scenes_graph_autotune(gg_scenes_graph *g, int trials, hipStream_t stream,
                              int *sweep_block, int *nlist_block, float *best_ms);
+/* (destroying or tuning a graph waits for its launches in flight) */
 void gg_scenes_graph_destroy(gg_scenes_graph *g);
 
 /* ---- batched scenes -------------------------------------------------------- */
@@ -579,6 +580,7 @@ int gg_batch_set_config(gg_batch *b, const gg_batch_config *cfg);
  * is unchanged on return; results never depend on the configuration. */
 int gg_batch_autotune(gg_batch *b, int trials, hipStream_t stream, gg_batch_config *best,
                       float *best_ms);
+/* (destroying, tuning or configuring waits for launches in flight) */
 void gg_batch_destroy(gg_batch *b);
 
 /* ---- captured step -------------------------------------------------------- */

@@ -89,6 +89,7 @@ hipError_t hipDeviceSynchronize() {
   for (ihipStream_t *s : std::set<ihipStream_t *>(streams)) wait_for(s);
   return hipSuccess;
 }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { return *g = new ihipGraph, hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) {

@@ -41,3 +41,8 @@ def _run(tmp_path, program, sources):
 def test_concurrent_learned_calls_wait_for_their_own_streams(tmp_path):
     r = _run(tmp_path, "side_stream.cpp", ["mlp.hip"])
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_graphs_are_not_released_with_launches_in_flight(tmp_path):
+    r = _run(tmp_path, "graphs.cpp", ["batch.hip", "scenes.hip"])
+    assert r.returncode == 0, r.stdout + r.stderr
