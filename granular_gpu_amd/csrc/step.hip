@@ -32,28 +32,10 @@
 #include "gg_device.hpp"
 #include "gg_internal.hpp"
 #include "grid_kernels.hpp"
+#include "list_quant.hpp"
 #include "profiler.hpp"
 
 namespace gg {
-
-// Positions for the list build's prefilter in 8 bytes: x, y, z in units of
-// L / 4096 modulo 2^16 (16 cells: differences inside a stencil are exact),
-// and minus the radius in units, rounded up, at most 4 cells.  Rounding moves
-// a coordinate difference by at most one unit plus what the product's own
-// rounding moves it (the margin of launch_nlist covers both).
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-constexpr int kQuantUnits = 4096;   // units per cell
-constexpr int kQuantMaxR = 16383;
-__device__ __forceinline__ int quant_up(float r, float per_unit) {
-  return (int)fminf(fmaxf(ceilf(r * per_unit) + 1.0f, 0.0f), (float)kQuantMaxR);
-}
-__device__ __forceinline__ uint2 quantise(const float4 &x, float per_unit) {
-  const unsigned int qx = (unsigned int)(int)rintf(x.x * per_unit);
-  const unsigned int qy = (unsigned int)(int)rintf(x.y * per_unit);
-  const unsigned int qz = (unsigned int)(int)rintf(x.z * per_unit);
-  const unsigned int r = (unsigned int)-quant_up(x.w, per_unit);
-  return make_uint2((qx & 0xffffu) | (qy << 16), (qz & 0xffffu) | (r << 16));
-}
 
 __global__ void __launch_bounds__(kBlock)
     k_permute_predict(int n, const int *__restrict__ raw, const int *__restrict__ key,
@@ -185,7 +167,21 @@ struct ListArgs {
   const unsigned int *__restrict__ bpart;
   int nbpart;
   unsigned int *__restrict__ bounds;
+  unsigned int *__restrict__ dirty;  // as the sweeps' marks
 };
+
+// Marks the cells whose stencils contain `cell` (sentinel: none) with a
+// displacement that the lists there have to allow for (non-negative floats,
+// and NaN above them, order like their bits).
+__device__ __forceinline__ void mark_cells(unsigned int *__restrict__ marks, const DevGrid &g,
+                                           int cell, unsigned int mark) {
+  if (cell < 0 || cell >= g.cx * g.cy * g.cz) return;
+  const int cz0 = cell % g.cz, cy0 = (cell / g.cz) % g.cy, cx0 = cell / (g.cz * g.cy);
+  for (int m = 0; m < 27; ++m) {
+    const int cc = stencil_cell(cx0, cy0, cz0, m, g);
+    if (cc >= 0) atomicMax(marks + cc, mark);
+  }
+}
 
 // Boundary candidates of i in scan order.
 __device__ __forceinline__ int boundary_list(const ListArgs &a, const DevGrid &g,
@@ -222,7 +218,10 @@ __device__ __forceinline__ int boundary_list(const ListArgs &a, const DevGrid &g
 // dot products, the sign shifted into a mask), where the exact test was 20
 // instructions and 16 bytes and kept the L1 return path 80% busy.  Its
 // survivors queue per lane in LDS and take the exact test in batches, in
-// order.  1M particles: 178 -> 130 us.
+// order.  A particle whose own limit does not fit the quantised form looks at
+// every candidate; one whose radius does not (4 cells) marks the cells around
+// it, so that nobody there uses a list that may lack it.  1M particles: 178
+// -> 134 us.
 constexpr int kListChunk = 24;  // candidates per mask (a row of three cells holds about as many)
 template <int BS, bool SCENES>
 __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
@@ -276,12 +275,8 @@ __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
     }
     queued = 0;
   };
-  const uint2 qi = quantise(si, a.per_unit);
-  int lim = quant_up(si.w + a.skin, a.per_unit) + a.margin;
-  lim = lim < kQuantMaxR ? lim : kQuantMaxR;
-  const s16x2 qxy = __builtin_bit_cast(s16x2, qi.x);
-  const s16x2 qz = __builtin_bit_cast(s16x2, (qi.y & 0xffffu) | ((unsigned int)lim << 16));
-  const s16x2 flip = {1, -1};
+  const QuantLimit ql = quant_limit(si, a.skin, a.per_unit, a.margin);
+  const unsigned int all = ql.all ? ~0u : 0u;
   // rows of three cells along z, each one index range, loaded a row ahead
   const int z0 = bz - 1 > 0 ? bz - 1 : 0;
   const int z1 = bz + 1 < g.cz - 1 ? bz + 1 : g.cz - 1;
@@ -312,16 +307,11 @@ __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
         for (int u = 0; u < 8; ++u) v[u] = a.xq[c0 + t + u];
         unsigned int m = 0u;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const s16x2 d = qxy - __builtin_bit_cast(s16x2, v[u].x);
-          const s16x2 w = qz - __builtin_bit_cast(s16x2, v[u].y);
-          const int e = __builtin_amdgcn_sdot2(
-              w, w * flip, __builtin_amdgcn_sdot2(d, d, 0, false), false);
-          m = __builtin_amdgcn_alignbit(m, (unsigned int)e, 31);
-        }
+        for (int u = 0; u < 8; ++u)
+          m = __builtin_amdgcn_alignbit(m, (unsigned int)quant_test(ql, v[u]), 31);
         mask |= m << (24 - t);  // candidate t + u in bit 31 - t - u
       }
-      if (cn > 0) mask &= ~0u << (32 - cn);
+      if (cn > 0) mask = (mask | all) & (~0u << (32 - cn));
       if (i >= c0 && i < c0 + cn) mask &= ~(0x80000000u >> (i - c0));
       if (__any(queued + (int)__popc(mask) > kListChunk)) flush();
       while (mask) {
@@ -335,7 +325,9 @@ __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
   flush();
   if (!live) return;
   const float4 bi = a.x[i];
-  a.meta[i] = make_int4(gc, bc, ext, hash_cell(bi.x, bi.y, bi.z, g));
+  const int cell = hash_cell(bi.x, bi.y, bi.z, g);
+  a.meta[i] = make_int4(gc, bc, ext, cell);
+  if (quant_large(si.w, a.per_unit)) mark_cells(a.dirty + lg.base, g, cell, 0x7f800000u);
   if (a.near) a.near[(size_t)kNearMax * a.sc.cap + i] = nc;
 }
 
@@ -482,19 +474,9 @@ __device__ __forceinline__ void sweep_store(const SweepArgs &a, int i, const flo
   const float3 m = mean_of(ab.x + ag.x, ab.y + ag.y, ab.z + ag.z, (float)(cnt > 1 ? cnt : 1));
   const float ox = oi.x + m.x, oy = oi.y + m.y, oz = oi.z + m.z;
   const float cum_new = oi.w + sqrt_any(m.x * m.x + m.y * m.y + m.z * m.z);
-  if (a.use_lists && !(cum_new < a.sc.half_valid) && cum_new != oi.w) {
-    const DevGrid &g = lg.g;
-    if (cell >= 0 && cell < g.cx * g.cy * g.cz) {
-      const int cz0 = cell % g.cz, cy0 = (cell / g.cz) % g.cy, cx0 = cell / (g.cz * g.cy);
-      // non-negative floats (and NaN above them) order like their bits
-      const unsigned int mark = __float_as_uint(cum_new);
-      unsigned int *marks = reinterpret_cast<unsigned int *>(a.dirty) + lg.base;
-      for (int m = 0; m < 27; ++m) {
-        const int cc = stencil_cell(cx0, cy0, cz0, m, g);
-        if (cc >= 0) atomicMax(marks + cc, mark);
-      }
-    }
-  }
+  if (a.use_lists && !(cum_new < a.sc.half_valid) && cum_new != oi.w)
+    mark_cells(reinterpret_cast<unsigned int *>(a.dirty) + lg.base, lg.g, cell,
+               __float_as_uint(cum_new));
   if (LAST_STAB) {
     const float4 d = a.d0[i];
     a.xb_out[i] = make_float4(bi.x + (ox - d.x), bi.y + (oy - d.y), bi.z + (oz - d.z), bi.w);
@@ -1299,16 +1281,14 @@ static int launch_nlist(int n, const float4 *xs, const int *cs, const int *bcs,
   a.sc = sweep_const(p, ws);
   a.skin = p->skin;
   a.per_unit = quant_per_unit(ws);
-  // a coordinate of q units is off by up to q 2^-23 before rounding; both
-  // ends of a difference, and rounding to whole units
-  const int cells = std::max(ws->grid.cx, std::max(ws->grid.cy, ws->grid.cz)) + 4;
-  a.margin = 4 + cells / 512;
+  a.margin = quant_margin(std::max(ws->grid.cx, std::max(ws->grid.cy, ws->grid.cz)));
   a.remap = (p->flags & GG_FLAG_NO_XCD_REMAP) ? 0 : 1;
   a.sv = sv ? *sv : SceneView{nullptr, nullptr, 0};
   a.gate = gate;
   a.bpart = nbpart > 0 ? at<unsigned int>(ws, L.bpart) : nullptr;
   a.nbpart = nbpart;
   a.bounds = at<unsigned int>(ws, L.bounds);
+  a.dirty = at<unsigned int>(ws, L.dirty);
   // (a block size asked for is k_nlist's; results do not depend on either)
   if (n <= kWideListMax && p->nlist_block == 0) {
     const int blocks = (n + 3) / 4 + (a.bpart ? 1 : 0);

@@ -1,0 +1,57 @@
+"""GPU tests of the list path against the oracle at the ends of its ranges:
+radii beyond what the list build's quantised test holds, frictions and masses
+outside the short arithmetic's domain, positions that are not finite."""
+import numpy as np
+import pytest
+import torch
+
+from granular_gpu_amd import scenes
+from oracle import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(s, steps=2, mu=(0.5, 0.4), nlist_block=0, sweep_block=0, flags=0):
+    from granular_gpu_amd.device import PlainSim
+    sim = PlainSim(s, stab=3, solver=5, mu_s=mu[0], mu_k=mu[1], flags=flags)
+    sim.params.nlist_block, sim.params.sweep_block = nlist_block, sweep_block
+    sim.step(steps)
+    gp, gv, _ = sim.host()
+    ctr = sim.view(8, 64, dtype=torch.int32, width=1).reshape(-1).cpu().numpy()
+    p = po.params_from(s, 3, 5, *mu)
+    bpos, bcs = po.sorted_boundary(s.boundary, s.cell_length, s.cells)
+    op, ov = po.plain_steps_f32(s.pos, s.vel, s.mass, bpos, bcs, p, steps)[:2]
+    return gp, gv, op, ov, ctr[1:9]
+
+
+def _equal(a, b):
+    return np.array_equal(a, b, equal_nan=True)
+
+
+def _with_large(side, cells_of_radius, count, seed):
+    """A lattice block with `count` particles of a radius of several cells,
+    each fast enough to cross some cells within the step: the lists are
+    built on the predicted positions, the cells on the present ones."""
+    s = scenes.plain_box(side, max(0.7, 0.022 * side), seed=seed)
+    rng = np.random.default_rng(seed)
+    k = rng.choice(s.n, count, replace=False)
+    s.mass[k] = (cells_of_radius * s.cell_length / 0.01) ** 3
+    d = rng.normal(size=(count, 3))
+    d *= rng.uniform(1.0, 4.5, (count, 1)) * s.cell_length / np.linalg.norm(d, axis=1)[:, None]
+    s.vel[k] = d / s.dt
+    return s
+
+
+@pytest.mark.parametrize("nlist_block,sweep_block", [(0, 0), (64, 0), (64, 64), (256, 256)])
+@pytest.mark.parametrize("cells_of_radius", [3.5, 4.1, 5.0, 9.0])
+def test_radii_of_several_cells(gpu, cells_of_radius, nlist_block, sweep_block):
+    s = _with_large(20, cells_of_radius, 20, seed=int(10 * cells_of_radius))
+    gp, gv, op, ov, _ = _run(s, 2, (0.5, 0.4), nlist_block, sweep_block)
+    assert _equal(gp, op) and _equal(gv, ov)
+
+
+def test_radii_of_several_cells_at_the_default_kernels_of_large_sets(gpu):
+    s = _with_large(41, 5.0, 12, seed=3)
+    assert s.n > 65536
+    gp, gv, op, ov, _ = _run(s, 1)
+    assert _equal(gp, op) and _equal(gv, ov)

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.skipif(not Path(HIPCC).exists(), reason="no hipcc")
 def _run(tmp_path, program, sources):
     """Links `program` with the host parts of the library's `sources` and the
     model, runs it."""
-    common = [HIPCC, "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-g", "-std=c++17",
+    common = [HIPCC, "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-g", "-std=c++17", "-ffp-contract=off",
               "-Wno-unused-command-line-argument", "-Xarch_host", "-fsanitize=address",
               f"-I{ROOT / 'include'}", f"-I{CSRC}", f"-I{HERE}"]
     objs = []
@@ -45,4 +45,9 @@ def test_concurrent_learned_calls_wait_for_their_own_streams(tmp_path):
 
 def test_graphs_are_not_released_with_launches_in_flight(tmp_path):
     r = _run(tmp_path, "graphs.cpp", ["batch.hip", "scenes.hip"])
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_quantised_list_test_loses_no_pair(tmp_path):
+    r = _run(tmp_path, "list_quant.cpp", [])
     assert r.returncode == 0, r.stdout + r.stderr
