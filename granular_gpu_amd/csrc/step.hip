@@ -27,8 +27,6 @@
 // scanning the stencil.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "gg_device.hpp"
 #include "gg_internal.hpp"
 #include "grid_kernels.hpp"
@@ -158,7 +156,6 @@ struct ListArgs {
   SweepConst sc;
   float skin;
   float per_unit;  // quantisation units per length
-  int margin;      // of the quantised test, in units
   int remap;
   SceneView sv;
   RefreshGate gate;
@@ -275,7 +272,10 @@ __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
     }
     queued = 0;
   };
-  const QuantLimit ql = quant_limit(si, a.skin, a.per_unit, a.margin);
+  // (positions are the particle's grid's: with scenes the workspace's grid is
+  // the concatenated tables, a million cells in a row)
+  const QuantLimit ql =
+      quant_limit(si, a.skin, a.per_unit, quant_margin(max(g.cx, max(g.cy, g.cz))));
   const unsigned int all = ql.all ? ~0u : 0u;
   // rows of three cells along z, each one index range, loaded a row ahead
   const int z0 = bz - 1 > 0 ? bz - 1 : 0;
@@ -1281,7 +1281,6 @@ static int launch_nlist(int n, const float4 *xs, const int *cs, const int *bcs,
   a.sc = sweep_const(p, ws);
   a.skin = p->skin;
   a.per_unit = quant_per_unit(ws);
-  a.margin = quant_margin(std::max(ws->grid.cx, std::max(ws->grid.cy, ws->grid.cz)));
   a.remap = (p->flags & GG_FLAG_NO_XCD_REMAP) ? 0 : 1;
   a.sv = sv ? *sv : SceneView{nullptr, nullptr, 0};
   a.gate = gate;

@@ -55,3 +55,28 @@ def test_radii_of_several_cells_at_the_default_kernels_of_large_sets(gpu):
     assert s.n > 65536
     gp, gv, op, ov, _ = _run(s, 1)
     assert _equal(gp, op) and _equal(gv, ov)
+
+
+def test_scenes_over_a_long_concatenated_table(gpu):
+    # ten scenes in grids of 60^3 cells: their tables are one of 2.2 million
+    # cells, their positions no larger than one scene's grid
+    from granular_gpu_amd.device import SceneBatch
+    scs, fr = [], []
+    for k in range(10):
+        s = scenes.plain_box(6 + k % 5, 2.4, seed=1 + k)
+        s.vel[:] = np.random.default_rng(k).normal(0.0, 0.5, s.vel.shape)
+        if k == 3:  # some in the grid's far corner
+            s.pos[::2] += np.float32(1.9)
+        scs.append(s)
+        fr.append((0.3 + 0.05 * k, 0.2 + 0.05 * k))
+    assert sum(c.cells[0] * c.cells[1] * c.cells[2] for c in scs) > 2_000_000
+    for block in (0, 64):
+        sb = SceneBatch(scs, fr)
+        sb.params.nlist_block = block
+        sb.step(6)
+        for k, s in enumerate(scs):
+            gp, gv, _ = sb.scene(k)
+            p = po.params_from(s, 3, 5, *fr[k])
+            bpos, bcs = po.sorted_boundary(s.boundary, s.cell_length, s.cells)
+            op, ov = po.plain_steps_f32(s.pos, s.vel, s.mass, bpos, bcs, p, 6)[:2]
+            assert _equal(gp, op) and _equal(gv, ov), (block, k)
