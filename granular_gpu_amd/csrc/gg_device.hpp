@@ -395,12 +395,14 @@ __device__ __forceinline__ bool granular_terms(const float4 &bi, const float4 &o
 // that meets operands outside the short sequences' domains (positions less
 // than 2^-48 apart but distinct, tangential displacements below 2^-48 or
 // above 2^20, rcp_refine's tie: one contact in 10^7) is evaluated again with
-// the full sequences.  Callers
-// keep list_fast's conditions (radii below 2^60, so a contact's d2 is finite;
-// mu_k 0 or in [2^-20, 2^20], so that mu_k delta is 0 or in [2^-92, 2^40]
-// since delta = rc - d is 0 or at least an ulp of d).  d2 = 0 (coincident
+// the full sequences.  Callers keep mu_k 0 or at least 2^-20, so that mu_k
+// delta is 0 or at least 2^-92 (delta = rc - d is 0 or at least an ulp of d).
+// Above 2^40 (large radii or coefficients, infinities) the quotient by a
+// displacement of at most 2^20 is far above 1 and comes out so, infinite or
+// NaN, all of which the minimum with 1 makes 1.  d2 = 0 (coincident
 // particles, and the particle itself in a padding slot) gives d = NaN, which
-// is no contact, as d > 0 demands.
+// is no contact, as d > 0 demands; so does an infinite d2, which no list
+// holds.
 constexpr unsigned int kSqrtFastMinBits = 0x0f800000u;  // 2^-96
 template <bool FRIC, bool STRICT>
 __device__ __forceinline__ bool fast_terms(float px, float py, float pz, float rx, float ry,

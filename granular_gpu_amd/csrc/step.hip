@@ -678,19 +678,17 @@ __device__ __forceinline__ void wave_stencil_seq(const SweepArgs &a, const Sweep
 }
 
 
-// The conditions of fast_terms on the particle and its neighbours (bounds[1]:
-// the step's largest radius) and on the friction.
+// fast_terms' condition on the friction (the same for a whole scene); lists
+// are evaluated by exact_list without it.
 template <bool FRIC>
-__device__ __forceinline__ bool list_fast(const SweepArgs &a, const SweepConst &sc, float r) {
-  const bool small = r + __uint_as_float(a.bounds[1]) < 0x1p60f && sc.rb + sc.rmin < 0x1p60f;
-  return small && (!FRIC || sc.mu_k == 0.0f || (sc.mu_k >= 0x1p-20f && sc.mu_k <= 0x1p20f));
+__device__ __forceinline__ bool fast_friction(const SweepConst &sc) {
+  return !FRIC || sc.mu_k == 0.0f || sc.mu_k >= 0x1p-20f;
 }
 
 // How a particle is evaluated in this sweep: 1 by its list, 2 by a scan of
 // the stencil of base (bx, by, bz), 3 not at all (no cell of the stencil lies
 // in the grid).  nc: entries of its near list, raised past kNearMax where
 // that is not usable.
-template <bool FRIC>
 __device__ __forceinline__ int sweep_mode(const SweepArgs &a, const SweepConst &sc,
                                           const LocalGrid &lg, const float4 &bi, const float4 &oi,
                                           const int4 &mt, int &bx, int &by, int &bz, int &nc) {
@@ -723,8 +721,7 @@ __device__ __forceinline__ int sweep_mode(const SweepArgs &a, const SweepConst &
       if (!(oi.w + fmaxf(__uint_as_float(mark), sc.half_valid) < sc.near_valid))
         nc = kNearMax + 1;
     }
-    list_ok = base_ok && moved_ok && mt.x <= sc.gmax && mt.y <= sc.bmax &&
-              list_fast<FRIC>(a, sc, bi.w);
+    list_ok = base_ok && moved_ok && mt.x <= sc.gmax && mt.y <= sc.bmax;
   }
   return list_ok ? 1 : (ext >= 0 ? 2 : 3);
 }
@@ -760,7 +757,7 @@ __device__ __forceinline__ void list_slots(const int *__restrict__ list, size_t 
 
 // A particle's list with the full square root and division sequences, for
 // operands outside the short ones' domains (a particle or two per million
-// and sweep).
+// and sweep, or every one under a friction outside them).
 template <bool FRIC>
 __device__ __forceinline__ void exact_list(const SweepArgs &a, const SweepConst &sc, int i,
                                            const float4 &bi, const float4 &oi, const int4 &mt,
@@ -848,7 +845,7 @@ __global__ void __launch_bounds__(BS, 5) k_sweep(SweepArgs a) {
         nc = a.near[(size_t)kNearMax * sc.cap + i];
       }
     }
-    mode = sweep_mode<FRIC>(a, sc, lg, bi, oi, mt, bx, by, bz, nc);
+    mode = sweep_mode(a, sc, lg, bi, oi, mt, bx, by, bz, nc);
   }
   const unsigned long long fb = __ballot(mode >= 2);
   if (a.stats && fb && lane == __ffsll((long long)fb) - 1) {
@@ -888,17 +885,18 @@ __global__ void __launch_bounds__(BS, 5) k_sweep(SweepArgs a) {
   float3 ab = make_float3(0.0f, 0.0f, 0.0f), ag = make_float3(0.0f, 0.0f, 0.0f);
   int nb = 0, ng = 0;
   if (mode == 1) {
-    bool redo = false;
+    bool redo = !fast_friction<FRIC>(sc);
+    const int bn = redo ? 0 : mt.y;
     // boundary candidates in list order, gathered four at a time (a particle
     // beside a dense boundary has dozens)
-    if (mt.y > 0) first_slots(a.blist + i, (size_t)sc.cap, sc.bmax, bj0);
-    list_slots(a.blist + i, (size_t)sc.cap, sc.bmax, mt.y, bj0, [&](const int (&k)[4], int t) {
+    if (bn > 0) first_slots(a.blist + i, (size_t)sc.cap, sc.bmax, bj0);
+    list_slots(a.blist + i, (size_t)sc.cap, sc.bmax, bn, bj0, [&](const int (&k)[4], int t) {
       float4 q[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) q[u] = a.bnd4[k[u]];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        if (t + u >= mt.y) continue;
+        if (t + u >= bn) continue;
         float3 c, f;
         if (fast_terms<FRIC, true>((bi.x - q[u].x) + oi.x, (bi.y - q[u].y) + oi.y,
                                    (bi.z - q[u].z) + oi.z, oi.x, oi.y, oi.z, rcb, sc.mu_s,
@@ -910,7 +908,7 @@ __global__ void __launch_bounds__(BS, 5) k_sweep(SweepArgs a) {
     });
     const bool near = nc <= kNearMax;
     const int *gl = near ? a.near + i : a.glist + i;
-    const int gn = near ? nc : mt.x;
+    const int gn = redo ? 0 : (near ? nc : mt.x);
     if (!near) first_slots(gl, (size_t)sc.cap, sc.gmax, gj0);
     list_slots(gl, (size_t)sc.cap, near ? kNearMax : sc.gmax, gn, gj0,
                [&](const int (&j)[4], int t) {
@@ -999,15 +997,16 @@ __global__ void __launch_bounds__(64) k_sweep_quad(SweepArgs a) {
 #pragma unroll
   for (int g = 0; g < 4; ++g) e[g] = 4 * g + sub < kNearMax ? a.near[(4 * g + sub) * cap + i] : i;
   int bx = 0, by = 0, bz = 0;
-  const int mode = live ? sweep_mode<FRIC>(a, sc, lg, bi, oi, mt, bx, by, bz, nc) : 0;
+  const int mode = live ? sweep_mode(a, sc, lg, bi, oi, mt, bx, by, bz, nc) : 0;
   const float rcb = sc.rb + fmaxf(bi.w, sc.rmin);
   float3 ab = make_float3(0.0f, 0.0f, 0.0f), ag = ab;
   int nb = 0, ng = 0;
-  bool redo = false;
+  bool redo = !fast_friction<FRIC>(sc);
+  const bool fast = mode == 1 && !redo;
   const float3 zero = ab;
   // contacts of the group in a ballot
   auto quad_count = [&](bool hit) { return __popc((unsigned int)(__ballot(hit) >> (lane & 60)) & 15u); };
-  const int bn = mode == 1 ? mt.y : 0;
+  const int bn = fast ? mt.y : 0;
   for (int t = 0; __any(t < bn); t += 4) {
     float3 c = zero, f = zero;
     bool hit = false;
@@ -1042,7 +1041,7 @@ __global__ void __launch_bounds__(64) k_sweep_quad(SweepArgs a) {
     add_quad<FRIC>(ag, c, f);
     ng += 2 * quad_count(hit);
   };
-  const int nn = mode == 1 && nc <= kNearMax ? nc : 0;
+  const int nn = fast && nc <= kNearMax ? nc : 0;
   if (__any(nn > 0)) {
     float4 b[4], o[4];
 #pragma unroll
@@ -1055,7 +1054,7 @@ __global__ void __launch_bounds__(64) k_sweep_quad(SweepArgs a) {
     for (int g = 0; g < 4; ++g)
       if (__any(4 * g < nn)) entry(4 * g + sub < nn, b[g], o[g]);
   }
-  const int gn = mode == 1 && nc > kNearMax ? mt.x : 0;
+  const int gn = fast && nc > kNearMax ? mt.x : 0;
   for (int t = 0; __any(t < gn); t += 4) {
     const bool on = t + sub < gn;
     const int j = on ? a.glist[(t + sub) * cap + i] : i;
@@ -1063,7 +1062,7 @@ __global__ void __launch_bounds__(64) k_sweep_quad(SweepArgs a) {
   }
   const bool again = quad_count(redo) != 0;
   if (sub == 0 && (mode == 1 || mode == 3)) {
-    if (again) exact_list<FRIC>(a, sc, i, bi, oi, mt, rcb, ab, ag, nb, ng);
+    if (again && mode == 1) exact_list<FRIC>(a, sc, i, bi, oi, mt, rcb, ab, ag, nb, ng);
     sweep_store<LAST_STAB>(a, i, bi, oi, ab, ag, nb + ng, mt.w, lg);
   }
   // the particles that scan their stencil, one after another

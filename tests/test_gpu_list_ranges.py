@@ -80,3 +80,46 @@ def test_scenes_over_a_long_concatenated_table(gpu):
             bpos, bcs = po.sorted_boundary(s.boundary, s.cell_length, s.cells)
             op, ov = po.plain_steps_f32(s.pos, s.vel, s.mass, bpos, bcs, p, 6)[:2]
             assert _equal(gp, op) and _equal(gv, ov), (block, k)
+
+
+def _pile(side, seed, shake=0.2):
+    """A block a little compressed: contacts everywhere, lists mostly valid."""
+    s = scenes.plain_box(side, max(0.7, 0.022 * side), seed=seed)
+    rng = np.random.default_rng(seed)
+    s.pos[:] = (0.15 + 0.97 * (s.pos - 0.15)).astype(np.float32)
+    s.vel[:] = rng.normal(0.0, shake, s.vel.shape)
+    return s
+
+
+# (0: four lanes a particle at this size, 64: one)
+@pytest.mark.parametrize("sweep_block", [0, 64])
+@pytest.mark.parametrize("mu", [(0.5, 1e-7), (0.0, 9e-7), (0.3, 1e-30), (0.5, 3e6), (0.0, 1e20),
+                                (0.5, -0.2), (1e25, 0.4)])
+def test_frictions_outside_the_short_division(gpu, mu, sweep_block):
+    s = _pile(16, 5)
+    usual = _run(s, 2, (0.5, 0.4), 0, sweep_block)[4]
+    gp, gv, op, ov, scans = _run(s, 2, mu, 0, sweep_block)
+    assert _equal(gp, op) and _equal(gv, ov)
+    # the lists are used as under an ordinary friction
+    assert usual.max() < s.n // 2 and scans.max() < s.n // 2
+
+
+@pytest.mark.parametrize("sweep_block", [0, 64])
+@pytest.mark.parametrize("mass", [np.nan, np.inf, -1.0, 0.0, 1e30])
+def test_one_odd_mass_leaves_the_others_their_lists(gpu, mass, sweep_block):
+    s = _pile(20, 6)
+    # beside a corner: an infinite radius reaches its whole stencil
+    k = int(np.argmin(np.abs(s.pos - s.pos.min(axis=0)).sum(axis=1)))
+    s.mass[k] = mass
+    gp, gv, op, ov, scans = _run(s, 1, (0.5, 0.4), 64 if sweep_block else 0, sweep_block)
+    assert _equal(gp, op) and _equal(gv, ov)
+    assert scans.max() < s.n // 2
+
+
+@pytest.mark.parametrize("nlist_block,sweep_block", [(0, 0), (64, 64)])
+def test_positions_and_velocities_that_are_not_finite(gpu, nlist_block, sweep_block):
+    s = _pile(16, 7)
+    s.pos[5], s.pos[77, 1], s.pos[900] = np.nan, np.inf, [1e30, -1e30, 3e38]
+    s.vel[11], s.vel[1234, 2], s.vel[2000] = np.nan, -np.inf, [1e25, 0.0, 0.0]
+    gp, gv, op, ov, _ = _run(s, 2, (0.5, 0.4), nlist_block, sweep_block)
+    assert _equal(gp, op) and _equal(gv, ov)
