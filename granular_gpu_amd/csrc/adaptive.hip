@@ -446,19 +446,26 @@ __global__ void __launch_bounds__(kBlock)
 // form chains and a round takes a quarter of them: of 80k claims 8k are left
 // after 6 rounds, 2k after 12, none after 36.  Up to kFinishMax claims the
 // block holds them in registers and their targets' owner and und in LDS, a
-// round costs about a microsecond where a launched one costs five; larger
-// lists go through global memory (atomics in L2, read around the L1).  und:
-// the last round's fold; pos: any array of n ints.  140k
-// particles, 80k claims: 950 us one after another, 70 us here.
+// round costs 3.6 us where a launched one costs five.  Longer
+// lists go through global memory (atomics in L2, read around the L1), each
+// round's undecided ones to the other list, until they fit on chip.  Where a
+// round decides fewer claims than would have been decided one after another
+// in its time (long chains, of which a round takes a link or two each), the
+// rest is taken in index order, so that the time stays linear in the claims:
+// about half a microsecond a claim and one per 1024 particles, against 4 for
+// a round on chip and 3 m / 1024 for one of m claims in memory.  und: the
+// last round's fold; pos, spare: any arrays of n ints.  140k particles, 80k
+// claims: 950 us one after another, 70 us here; 1M particles of a jittered
+// lattice, marking in all: 35.5 ms, now 1.7; 300 chains of 1000: 101, 125.
 constexpr int kFinishPer = 4, kFinishMax = 1024 * kFinishPer;
+constexpr int kFinishSlow = 128;
 __global__ void __launch_bounds__(1024)
-    k_merge_finish(const int *__restrict__ list, const int *__restrict__ left,
-                   const int *__restrict__ cand, int *state, int *owner, int *und, int *pos,
+    k_merge_finish(int n, int *list, const int *__restrict__ left, const int *__restrict__ cand,
+                   int *state, int *owner, int *und, int *pos, int *spare,
                    const int *__restrict__ surf, const float *__restrict__ sd, MergeRules R,
                    const float *__restrict__ rs) {
   __shared__ int open, own_s[kFinishMax], und_s[kFinishMax];
-  const int m = *left;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
   auto load = [](const int *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
@@ -466,6 +473,43 @@ __global__ void __launch_bounds__(1024)
     __builtin_amdgcn_s_waitcnt(0);  // this wave's stores and atomics have been performed
     __syncthreads();
   };
+  int m = *left;
+  while (m > kFinishMax) {
+    if (tid == 0) open = 0;
+    __syncthreads();
+    for (int b = 0; b < m; b += 1024) {
+      int st = M_NONE, i = 0;
+      if (b + tid < m) {
+        i = list[b + tid];
+        const int c = cand[i];
+        st = merge_decision(i, load(&owner[i]), load(&owner[c]), load(&und[i]), load(&und[c]),
+                            deep_at(i, surf, sd, R, rs), deep_at(c, surf, sd, R, rs));
+        if (st != M_UND) state[i] = st;
+        if (st == M_SUCCESS || st == M_PARTNER_LOCK) atomicMin(&owner[c], i);
+      }
+      converge();
+      const unsigned long long u = __ballot(st == M_UND);
+      int at = 0;
+      if (lane == 0 && u) at = atomicAdd(&open, (int)__popcll(u));
+      at = __shfl(at, 0, 64);
+      if (st == M_UND) spare[at + (int)__popcll(u & ((1ull << lane) - 1ull))] = i;
+      converge();
+    }
+    meet();
+    const int todo = open;
+    for (int k = tid; k < m; k += 1024) atomicExch(&und[cand[list[k]]], INT_MAX);
+    meet();
+    if (todo > kFinishMax && (m - todo) < m / kFinishSlow) break;
+    for (int k = tid; k < todo; k += 1024) {
+      const int i = spare[k];
+      atomicMin(&und[cand[i]], i);
+    }
+    meet();
+    int *const t = list;
+    list = spare;
+    spare = t;
+    m = todo;
+  }
   if (m <= kFinishMax) {
     // a target's slot: the list position of its lowest undecided claimer
     for (int k = tid; k < m; k += 1024) atomicExch(&pos[list[k]], k);
@@ -478,19 +522,20 @@ __global__ void __launch_bounds__(1024)
       st[q] = M_NONE;
       if (k >= m) continue;
       const int i = list[k], c = cand[i];
-      const int ui = und[i], uc = und[c];
+      const int ui = load(&und[i]), uc = load(&und[c]);
       idx[q] = i;
       st[q] = M_UND;
       sc[q] = load(&pos[uc]);
       si[q] = ui == INT_MAX ? -1 : load(&pos[ui]);
-      own0[q] = owner[i];  // stays while nothing undecided claims i
+      own0[q] = load(&owner[i]);  // stays while nothing undecided claims i
       deep_i[q] = deep_at(i, surf, sd, R, rs);
       deep_c[q] = deep_at(c, surf, sd, R, rs);
-      own_s[sc[q]] = owner[c];
+      own_s[sc[q]] = load(&owner[c]);
       und_s[sc[q]] = uc;
     }
     meet();
-    for (int todo = m; todo > 0;) {
+    int todo = m;
+    for (bool slow = false; todo > 0 && !slow;) {
       if (tid == 0) open = 0;
 #pragma unroll
       for (int q = 0; q < kFinishPer; ++q) {
@@ -513,41 +558,54 @@ __global__ void __launch_bounds__(1024)
       }
       if (mine) atomicAdd(&open, mine);
       __syncthreads();
+      const int decided = todo - open;
       todo = open;
+      slow = 4ll * todo > (long long)decided * (todo / 2 + n / 1024);
       __syncthreads();
     }
 #pragma unroll
-    for (int q = 0; q < kFinishPer; ++q)
-      if (tid + 1024 * q < m) state[idx[q]] = st[q];
-    return;
+    for (int q = 0; q < kFinishPer; ++q) {
+      if (tid + 1024 * q >= m) continue;
+      state[idx[q]] = st[q];
+      if (todo > 0) atomicMin(&owner[cand[idx[q]]], own_s[sc[q]]);
+    }
+    if (todo == 0) return;
+    meet();
   }
-  for (int todo = m; todo > 0;) {
-    if (tid == 0) open = 0;
-    for (int k = tid; k < m; k += 1024) {
-      const int i = list[k];
-      if (state[i] != M_UND) continue;
+  // index order: the block lists the undecided of 1024 particles, their
+  // targets and rules, one thread decides them
+  int *const idx = own_s, *const target = own_s + 1024, *const rule = own_s + 2048,
+             *const count = und_s;
+  for (int b = 0; b < n; b += 1024) {
+    const int i = b + tid;
+    const bool f = i < n && state[i] == M_UND;
+    const unsigned long long u = __ballot(f);
+    if (lane == 0) count[tid >> 6] = (int)__popcll(u);
+    __syncthreads();
+    int at = 0, total = 0;
+    for (int w = 0; w < 16; ++w) {
+      if (w == tid >> 6) at = total;
+      total += count[w];
+    }
+    if (f) {
+      const int k = at + (int)__popcll(u & ((1ull << lane) - 1ull));
       const int c = cand[i];
-      const int st = merge_decision(i, load(&owner[i]), load(&owner[c]), load(&und[i]),
-                                    load(&und[c]), deep_at(i, surf, sd, R, rs),
-                                    deep_at(c, surf, sd, R, rs));
-      if (st == M_UND) continue;
-      state[i] = st;
-      if (st == M_SUCCESS || st == M_PARTNER_LOCK) atomicMin(&owner[c], i);
+      idx[k] = i;
+      target[k] = c;
+      rule[k] = (deep_at(i, surf, sd, R, rs) ? 1 : 0) | (deep_at(c, surf, sd, R, rs) ? 2 : 0);
     }
-    meet();
-    for (int k = tid; k < m; k += 1024) atomicExch(&und[cand[list[k]]], INT_MAX);
-    meet();
-    int mine = 0;
-    for (int k = tid; k < m; k += 1024) {
-      const int i = list[k];
-      if (state[i] != M_UND) continue;
-      atomicMin(&und[cand[i]], i);
-      ++mine;
+    __syncthreads();
+    if (tid == 0) {
+      for (int k = 0; k < total; ++k) {
+        const int c = target[k];
+        const int st = merge_decision(idx[k], load(&owner[idx[k]]), load(&owner[c]), INT_MAX,
+                                      INT_MAX, (rule[k] & 1) != 0, (rule[k] & 2) != 0);
+        state[idx[k]] = st;
+        if (st == M_SUCCESS || st == M_PARTNER_LOCK) atomicMin(&owner[c], idx[k]);
+        __builtin_amdgcn_s_waitcnt(0);  // the next claim reads owner
+      }
     }
-    if (mine) atomicAdd(&open, mine);
-    meet();
-    todo = open;
-    meet();
+    __syncthreads();
   }
 }
 
@@ -894,9 +952,9 @@ static int merge_mark_rules(gg_particles *set, gg_adaptive *ad, const int *cell_
                                              r == rounds - 1 ? list : nullptr, left);
     GG_LAUNCH_CHECK();
   }
-  k_merge_finish<<<1, 1024, 0, stream>>>(list, left, cand, state, owner, und[rounds % 3],
-                                         und[(rounds + 1) % 3], set->surface,
-                                         set->surface_distance, R, rs);
+  k_merge_finish<<<1, 1024, 0, stream>>>(n, list, left, cand, state, owner, und[rounds % 3],
+                                         und[(rounds + 1) % 3], und[(rounds + 2) % 3],
+                                         set->surface, set->surface_distance, R, rs);
   GG_LAUNCH_CHECK();
   k_merge_apply<<<nb, kBlock, 0, stream>>>(n, cand, state, dens, set->mass,
                                            reinterpret_cast<const float *>(set->vel), ad->remove,
