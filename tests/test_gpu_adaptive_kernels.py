@@ -93,6 +93,30 @@ def test_stencil_passes_equal_oracle(gpu, n, crowd):
         assert np.array_equal(a, b)
 
 
+def test_positions_and_masses_that_are_not_finite(gpu):
+    from granular_gpu_amd import _lib
+    from granular_gpu_amd.device import _ptr, _stream
+    s = _cloud(900, 4, 0.4)
+    s.pos[3], s.pos[40, 1], s.pos[500] = np.nan, np.inf, [1e30, -1e30, 0.1]
+    s.mass[[7, 300, 700, 701]] = [np.nan, np.inf, -1.0, 0.0]
+    sim, pos, vel, mass, cs = _sorted_sim(s)
+    n = s.n
+    p, lib = po.params_from(s, 3, 5), po.load()
+    _lib.check("gg_surface", sim.lib.gg_surface(C.byref(sim.set), _ptr(sim.cs),
+                                                C.byref(sim.params), C.byref(sim.ws), _stream()))
+    _lib.check("gg_surface_distance", sim.lib.gg_surface_distance(
+        C.byref(sim.set), _ptr(sim.cs), C.byref(sim.ws), _stream()))
+    cover, surf, sd = np.zeros((n, 3), np.float32), np.zeros(n, np.int32), np.zeros(n, np.float32)
+    lib.oracle_surface(n, pos.reshape(-1), mass, cs, p, cover.reshape(-1), surf)
+    lib.oracle_surface_distance(n, pos.reshape(-1), surf, cs, p, sd)
+    assert np.array_equal(sim.surface[:n].cpu().numpy(), surf)
+    assert np.array_equal(sim.sd[:n].cpu().numpy(), sd)
+    surf[:], sd[:] = 0, 1e5
+    sim.surface[:n], sim.sd[:n] = 0, 1e5
+    for a, b in zip(_mark(sim, 16.0), _oracle_mark(s, pos, vel, mass, surf, sd, cs, 16.0)):
+        assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
+
+
 # the last four leave the launched rounds some hundred thousand claims: in
 # chains so long that the finisher goes over to index order at once, after some
 # rounds, or never

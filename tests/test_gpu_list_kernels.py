@@ -85,3 +85,24 @@ def test_steps_equal_oracle(gpu, kind, n, seed, mu):
     bpos, bcs = po.sorted_boundary(s.boundary, s.cell_length, s.cells)
     op, ov = po.plain_steps_f32(s.pos, s.vel, s.mass, bpos, bcs, p, 3)[:2]
     assert np.array_equal(gp, op) and np.array_equal(gv, ov)
+
+
+@pytest.mark.parametrize("kind,n,seed", CASES)
+@pytest.mark.parametrize("nlist_block,sweep_block", [(64, 64), (256, 256), (0, 64), (64, 0)])
+@pytest.mark.parametrize("refresh", [False, True])
+def test_every_pair_of_kernels_equals_oracle(gpu, kind, n, seed, nlist_block, sweep_block,
+                                             refresh):
+    # each list build (64, 256: one lane a particle, as for large sets) with
+    # each sweep, near lists included; refreshed within the step too
+    from granular_gpu_amd._lib import GG_FLAG_LIST_REFRESH
+    from granular_gpu_amd.device import PlainSim
+    s = _scene(kind, n, seed)
+    sim = PlainSim(s, stab=3, solver=5, mu_s=0.5, mu_k=0.4,
+                   flags=GG_FLAG_LIST_REFRESH if refresh else 0)
+    sim.params.nlist_block, sim.params.sweep_block = nlist_block, sweep_block
+    sim.step(3)
+    gp, gv, _ = sim.host()
+    p = po.params_from(s, 3, 5, 0.5, 0.4)
+    bpos, bcs = po.sorted_boundary(s.boundary, s.cell_length, s.cells)
+    op, ov = po.plain_steps_f32(s.pos, s.vel, s.mass, bpos, bcs, p, 3)[:2]
+    assert np.array_equal(gp, op) and np.array_equal(gv, ov)
