@@ -484,24 +484,23 @@ __global__ void __launch_bounds__(256)
 // chunk, each with an LDS round trip and at most 8 dependent MFMAs), not
 // memory or MFMA rate, so the layers share one launch: a gradient was 23
 // launches (a strided 2-byte GEMM per product, bias / ReLU / mask / loss /
-// column-sum passes between them) and is 2.  Measured: a gradient, an Adam
-// update and a quarter of a forward over 2,048 rows for 512 samples 216 -> 34
-// us (kernels 18.6 + 4.0 + 3.4 + 11.5 / 4; the rest is the host's launches),
-// with a forward over 8,192 samples 1371 -> 51 us (36 + 5 + 4 + 12).
+// column-sum passes between them) and is 2.  Measured: four times a gradient
+// and an Adam update over 512 samples and a forward over 2,048 rows 865 ->
+// 109 us (kernels 14.4 + 3.9 + 3.4, 7.5; the rest is the host's launches),
+// one over 8,192 samples and rows 1369 -> 40 us (30 + 5 + 4 + 8).
 //
-// Operands are consecutive elements of one row, so every product reads rows
-// whose contraction index is contiguous.  A hidden layer is stored twice in
-// LDS for that, [sample][feature] (the next layer's contraction) and
-// [feature][sample] (the weight gradient's).  Wave w owns features 16 w ..
-// 16 w + 15 of every hidden layer.
+// v_mfma_f32_16x16x32_bf16 with k = 8 q + e for element e of lane (c, q) in
+// both operands: an operand is 8 consecutive elements of one row, so every
+// product reads rows whose contraction index is contiguous.  A hidden layer
+// is stored twice in LDS for that, [sample][feature] (the next layer's
+// contraction) and [feature][sample] (the weight gradient's).  Wave w owns
+// features 16 w .. 16 w + 15 of every hidden layer.
 //
-// The products between layers take v_mfma_f32_16x16x16_bf16 in ascending k,
-// the bias after the sum: the order and the shape decide the last bits of
-// the values that are rounded to bfloat16, and a flipped rounding moves a
-// gradient by far more (the 16x16x32 shape: 1e-4 of a layer's norm) than
-// the order of a weight gradient's FP32 sums does (1e-6).  The wider shape
-// would take 30 us instead of 36 for 8,192 samples.  The weight gradients,
-// which are not rounded, have it.
+// Every product is summed in ascending k with the bias added last: the order
+// decides the last bits of the values that are rounded to bfloat16, and a
+// flipped rounding changes an output by up to 2^-8 of a hidden value.  (Sums
+// in steps of 32 and of 16 features came out the same bits; starting at the
+// bias, or in the inference kernel's order of features, does not.)
 constexpr int kChunk = 32;           // samples per pass = one MFMA k-step of the weight gradient
 constexpr int kRowF = kHid + 8;      // [sample][feature] row, padded (16-byte rows, no bank pile-up)
 constexpr int kRowS = kChunk + 8;    // [feature][sample] row, padded the same way
@@ -509,29 +508,30 @@ constexpr int kGradWaves = 8;
 constexpr int kPartial = 49152 + 416;  // floats of one block's partial gradient
 constexpr int kGradBlocks = 128;       // at most this many partial gradients
 
-// 4 bfloat16 / 4 floats from memory of any element alignment.
+// 8 bfloat16 / 4 floats from memory of any element alignment.
+typedef bf16x8 bf16x8_u __attribute__((aligned(2)));
 typedef bf16x4 bf16x4_u __attribute__((aligned(2)));
 typedef f32x4 f32x4_u __attribute__((aligned(4)));
-__device__ __forceinline__ bf16x4 ld4(const uint16_t *p) {
-  return *reinterpret_cast<const bf16x4_u *>(p);
+__device__ __forceinline__ bf16x8 ld8(const uint16_t *p) {
+  return *reinterpret_cast<const bf16x8_u *>(p);
+}
+
+// Row n of a row-major matrix of 32 KS columns as the KS operands of lane
+// quarter q.
+template <int KS>
+__device__ __forceinline__ void ld_row(const uint16_t *__restrict__ row, int q,
+                                       bf16x8 (&v)[KS]) {
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) v[ks] = ld8(row + 32 * ks + 8 * q);
 }
 
 // Element e: W[n0 + e][k] of a row-major matrix of K columns (a weight
 // fragment whose contraction runs over rows).
-__device__ __forceinline__ bf16x4 ld4_rows(const uint16_t *__restrict__ W, int K, int n0, int k) {
-  bf16x4 v;
+__device__ __forceinline__ bf16x8 ld8_rows(const uint16_t *__restrict__ W, int K, int n0, int k) {
+  bf16x8 v;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = (short)W[(n0 + e) * K + k];
+  for (int e = 0; e < 8; ++e) v[e] = (short)W[(n0 + e) * K + k];
   return v;
-}
-
-// Row n of a row-major matrix of 16 KS columns as the KS operands of lane
-// quarter q.
-template <int KS>
-__device__ __forceinline__ void ld_row(const uint16_t *__restrict__ row, int q,
-                                       bf16x4 (&v)[KS]) {
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) v[ks] = ld4(row + 16 * ks + 4 * q);
 }
 
 __device__ __forceinline__ bf16x4 to_bf16x4(const f32x4 &v) {
@@ -550,17 +550,17 @@ __device__ __forceinline__ void put_tile(uint16_t *bf, uint16_t *fb, int f0, int
 
 // Sum over KS k-steps of a[ks] times one [sample][feature] row per lane.
 template <int KS>
-__device__ __forceinline__ f32x4 row_product(const bf16x4 (&a)[KS], const uint16_t *row, int q) {
+__device__ __forceinline__ f32x4 row_product(const bf16x8 (&a)[KS], const uint16_t *row, int q) {
   f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
-    z = mfma16(a[ks], *reinterpret_cast<const bf16x4 *>(row + 16 * ks + 4 * q), z);
+    z = mfma32(a[ks], *reinterpret_cast<const bf16x8 *>(row + 32 * ks + 8 * q), z);
   return z;
 }
 
 // The same for both sample tiles of a chunk.
 template <int KS>
-__device__ __forceinline__ void rows_product(const bf16x4 (&a)[KS], const uint16_t *bf, int c,
+__device__ __forceinline__ void rows_product(const bf16x8 (&a)[KS], const uint16_t *bf, int c,
                                              int q, f32x4 (&out)[2]) {
 #pragma unroll
   for (int s = 0; s < 2; ++s) out[s] = row_product<KS>(a, bf + (16 * s + c) * kRowF, q);
@@ -576,14 +576,6 @@ __device__ __forceinline__ void weight_product(const uint16_t *gs, const uint16_
   for (int t = 0; t < T; ++t)
     acc[t] = mfma32(a, *reinterpret_cast<const bf16x8 *>(hs + (16 * t + c) * kRowS + 8 * q),
                     acc[t]);
-}
-
-// The features of sample smp (zeros past the batch) as layer 1's operands.
-__device__ __forceinline__ void load_rows(const uint16_t *__restrict__ x, int smp, int B, int q,
-                                          bf16x4 (&v)[6]) {
-#pragma unroll
-  for (int ks = 0; ks < 6; ++ks) v[ks] = bf16x4{0, 0, 0, 0};
-  if (smp < B) ld_row<6>(x + (size_t)smp * kIn, q, v);
 }
 
 struct GradArgs {
@@ -609,12 +601,12 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_mlp_grad(GradArgs a) {
   const float scale = 2.0f / (float)(kOut * a.B);
   // weight fragments of the way back (contraction over rows: 2-byte
   // gathers), loaded once
-  bf16x4 t4[2], t3[8], t2[8];
+  bf16x8 t4[1], t3[4], t2[4];
+  t4[0] = ld8_rows(a.w + kWOff4, kHid, 8 * q, 16 * w + c);
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    if (ks < 2) t4[ks] = ld4_rows(a.w + kWOff4, kHid, 16 * ks + 4 * q, 16 * w + c);
-    t3[ks] = ld4_rows(a.w + kWOff3, kHid, 16 * ks + 4 * q, 16 * w + c);
-    t2[ks] = ld4_rows(a.w + kWOff2, kHid, 16 * ks + 4 * q, 16 * w + c);
+  for (int ks = 0; ks < 4; ++ks) {
+    t3[ks] = ld8_rows(a.w + kWOff3, kHid, 32 * ks + 8 * q, 16 * w + c);
+    t2[ks] = ld8_rows(a.w + kWOff2, kHid, 32 * ks + 8 * q, 16 * w + c);
   }
   f32x4 w1[6], w2[8], w3[8], w4[2];  // weight gradients: tiles of rows 16 w (w4: columns 16 w)
   f32x4 b1 = {0.0f, 0.0f, 0.0f, 0.0f}, b2 = b1, b3 = b1, b4[2] = {b1, b1};
@@ -627,6 +619,7 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_mlp_grad(GradArgs a) {
   const int chunks = (a.B + kChunk - 1) / kChunk;
   for (int ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
     const int base = ch * kChunk;
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     f32x4 z[2];
     unsigned int mask[3] = {0u, 0u, 0u};  // bit 4 s + e of layer l: Z > 0
     // hidden layer l's tile from its product z: bias, ReLU, both layouts
@@ -645,35 +638,45 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_mlp_grad(GradArgs a) {
     };
     // layer 1 from x (rows past the batch: zeros)
     {
-      bf16x4 wf[6], xf[2][6];
-      ld_row<6>(a.w + kWOff1 + (16 * w + c) * kIn, q, wf);
+      bf16x8 wf[3], xf[2][3];
 #pragma unroll
-      for (int s = 0; s < 2; ++s) load_rows(a.x, base + 16 * s + c, a.B, q, xf[s]);
+      for (int ks = 0; ks < 3; ++ks) {
+        wf[ks] = ld8(a.w + kWOff1 + (16 * w + c) * kIn + 32 * ks + 8 * q);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int smp = base + 16 * s + c;
+          xf[s][ks] = smp < a.B ? ld8(a.x + (size_t)smp * kIn + 32 * ks + 8 * q) : zero8;
+        }
+      }
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         z[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int ks = 0; ks < 6; ++ks) {
-          z[s] = mfma16(wf[ks], xf[s][ks], z[s]);
-          // wave (6 s + ks) % 8 keeps this fragment's x^T
-          if (w == (6 * s + ks) % kGradWaves) {
+        for (int ks = 0; ks < 3; ++ks) {
+          z[s] = mfma32(wf[ks], xf[s][ks], z[s]);
+          // wave 3 s + ks keeps this fragment's x^T
+          if (w == 3 * s + ks) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              xs[(16 * ks + 4 * q + e) * kRowS + 16 * s + c] = (uint16_t)xf[s][ks][e];
+            for (int e = 0; e < 8; ++e)
+              xs[(32 * ks + 8 * q + e) * kRowS + 16 * s + c] = (uint16_t)xf[s][ks][e];
           }
         }
       }
       activate(0, rows[0], hs[0]);
     }
     {
-      bf16x4 wf[8];
-      ld_row<8>(a.w + kWOff2 + (16 * w + c) * kHid, q, wf);
+      bf16x8 wf[4];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        wf[ks] = ld8(a.w + kWOff2 + (16 * w + c) * kHid + 32 * ks + 8 * q);
       __syncthreads();
-      rows_product<8>(wf, rows[0], c, q, z);
+      rows_product<4>(wf, rows[0], c, q, z);
       activate(1, rows[1], hs[1]);
-      ld_row<8>(a.w + kWOff3 + (16 * w + c) * kHid, q, wf);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        wf[ks] = ld8(a.w + kWOff3 + (16 * w + c) * kHid + 32 * ks + 8 * q);
       __syncthreads();
-      rows_product<8>(wf, rows[1], c, q, z);
+      rows_product<4>(wf, rows[1], c, q, z);
       activate(2, rows[0], hs[2]);
       __syncthreads();
     }
@@ -683,9 +686,9 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_mlp_grad(GradArgs a) {
       float s2 = 0.0f;
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        bf16x4 wf[8];
-        ld_row<8>(a.w + kWOff4 + (16 * t + c) * kHid, q, wf);
-        const f32x4 y = row_product<8>(wf, rows[0] + (16 * w + c) * kRowF, q);
+        bf16x8 wf[4];
+        ld_row<4>(a.w + kWOff4 + (16 * t + c) * kHid, q, wf);
+        const f32x4 y = row_product<4>(wf, rows[0] + (16 * w + c) * kRowF, q);
         f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f};
         if (smp < a.B && 16 * t + 4 * q < kOut) {
           const f32x4 e = (y + *reinterpret_cast<const f32x4_u *>(a.bias + kBOff4 + 16 * t +
@@ -724,15 +727,15 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_mlp_grad(GradArgs a) {
         w4[t] = mfma32(*reinterpret_cast<const bf16x8 *>(gs[0] + (16 * t + c) * kRowS + 8 * q),
                        hv, w4[t]);
     }
-    rows_product<2>(t4, rows[1], c, q, z);
+    rows_product<1>(t4, rows[1], c, q, z);
     backward(2, b3, rows[0], gs[1]);
     __syncthreads();
     weight_product<8>(gs[1], hs[1], 16 * w, c, q, w3);
-    rows_product<8>(t3, rows[0], c, q, z);
+    rows_product<4>(t3, rows[0], c, q, z);
     backward(1, b2, rows[1], gs[0]);
     __syncthreads();
     weight_product<8>(gs[0], hs[0], 16 * w, c, q, w2);
-    rows_product<8>(t2, rows[1], c, q, z);
+    rows_product<4>(t2, rows[1], c, q, z);
     backward(0, b1, nullptr, gs[1]);
     __syncthreads();
     weight_product<6>(gs[1], xs, 16 * w, c, q, w1);
@@ -796,11 +799,11 @@ __global__ void __launch_bounds__(64 * kGradWaves)
   const int c = lane & 15, q = lane >> 4;
   const int f0 = 16 * w + 4 * q;
   const int so = w & 1, to = (w >> 1) & 1;  // this wave's output tile (waves 0..3)
-  bf16x4 wf1[6], wf2[8], wf3[8], wf4[8];
-  ld_row<6>(wts + kWOff1 + (16 * w + c) * kIn, q, wf1);
-  ld_row<8>(wts + kWOff2 + (16 * w + c) * kHid, q, wf2);
-  ld_row<8>(wts + kWOff3 + (16 * w + c) * kHid, q, wf3);
-  ld_row<8>(wts + kWOff4 + (16 * to + c) * kHid, q, wf4);
+  bf16x8 wf1[3], wf2[4], wf3[4], wf4[4];
+  ld_row<3>(wts + kWOff1 + (16 * w + c) * kIn, q, wf1);
+  ld_row<4>(wts + kWOff2 + (16 * w + c) * kHid, q, wf2);
+  ld_row<4>(wts + kWOff3 + (16 * w + c) * kHid, q, wf3);
+  ld_row<4>(wts + kWOff4 + (16 * to + c) * kHid, q, wf4);
   const int chunks = (n + kChunk - 1) / kChunk;
   for (int ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
     const int base = ch * kChunk;
@@ -817,23 +820,26 @@ __global__ void __launch_bounds__(64 * kGradWaves)
     };
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      bf16x4 xf[6];
-      load_rows(x, base + 16 * s + c, n, q, xf);
+      const int smp = base + 16 * s + c;
+      bf16x8 xf[3];
+#pragma unroll
+      for (int ks = 0; ks < 3; ++ks) xf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (smp < n) ld_row<3>(x + (size_t)smp * kIn, q, xf);
       z[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int ks = 0; ks < 6; ++ks) z[s] = mfma16(wf1[ks], xf[ks], z[s]);
+      for (int ks = 0; ks < 3; ++ks) z[s] = mfma32(wf1[ks], xf[ks], z[s]);
     }
     activate(0, rows[0]);
     __syncthreads();
-    rows_product<8>(wf2, rows[0], c, q, z);
+    rows_product<4>(wf2, rows[0], c, q, z);
     activate(1, rows[1]);
     __syncthreads();
-    rows_product<8>(wf3, rows[1], c, q, z);
+    rows_product<4>(wf3, rows[1], c, q, z);
     activate(2, rows[0]);
     __syncthreads();
     if (w < 4) {
       const int smp = base + 16 * so + c, o = 16 * to + 4 * q;
-      const f32x4 y = row_product<8>(wf4, rows[0] + (16 * so + c) * kRowF, q);
+      const f32x4 y = row_product<4>(wf4, rows[0] + (16 * so + c) * kRowF, q);
       if (smp < n && o < kOut) {
         const f32x4 v = y + *reinterpret_cast<const f32x4_u *>(bias + kBOff4 + o);
         *reinterpret_cast<f32x4_u *>(y_out + (size_t)smp * kOut + o) = v;
