@@ -129,7 +129,7 @@ __device__ __forceinline__ unsigned int group_ballot(const Group &G, bool p) {
 }
 
 // The group's neighbours found so far, in scan order, in LDS.
-constexpr int kHits = 128;
+constexpr int kHits = 320;
 struct Hits {
   int *list;   // kHits entries of this group
   int count;   // the same on every lane of the group
@@ -173,8 +173,10 @@ __global__ void __launch_bounds__(kBlock) k_radius_surface(int n, const float *_
 // <=> n <= 5 or no neighbour inside the pi/3 cone around the normalised cover
 // vector (acos(d) <= pi/3 tested as d >= 0.5).  The scan keeps the neighbours
 // (some 30 of hundreds of candidates) in LDS for the vote; only a particle
-// with more than fit scans twice.  16 lanes and one scan instead of
-// two: 140k particles, 176 + 162 -> 96 us.
+// with more than fit scans twice.  16 lanes and one scan instead of two: 140k
+// particles, 176 + 162 -> 95 us; 1.2M, 894 -> 711; 3M in a funnel, 2627 ->
+// 1890; 1.9M of 200 to 1600 candidates each, 3161 -> 2655 (lists of 128, which
+// many of them overflow: 3590).
 __global__ void __launch_bounds__(64)
     k_cover_surface(int n, const float *__restrict__ pos, const float *__restrict__ rs,
                     const int *__restrict__ cs, DevGrid g, int *__restrict__ surf) {
@@ -296,6 +298,50 @@ __global__ void __launch_bounds__(64)
     best = v < best ? v : best;
   }
   if (live && G.sub == 0) sd[i] = here ? 0.0f : best;
+}
+
+// The same with one lane per particle, for sets that fill the chip with it:
+// neighbouring lanes test the same candidates, so a wave's load is a cache
+// line or two where 16 lanes per particle read some twenty, and without
+// neighbours to keep the loads are what the pass takes.  Beds of 23 a cell: up
+// to 204k particles 16 lanes (54, one 72 us), 304k the same (85, 81), 1.2M one
+// (293, 248); 1.9M of 200 to 1600 candidates each 1262, 735.
+constexpr int kGroupDistanceMax = 262144;
+__global__ void __launch_bounds__(kBlock)
+    k_surface_distance_lane(int n, const float *__restrict__ pos, const int *__restrict__ surf,
+                            const int *__restrict__ cs, DevGrid g, float *__restrict__ sd) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (surf[i] == 1) {
+    sd[i] = 0.0f;
+    return;
+  }
+  const Packed3 x = ld3(pos, i);
+  float best = 100000.0f;
+  auto test = [&](int j, const Packed3 &q, int sj) {
+    const float dx = x.x - q.x, dy = x.y - q.y, dz = x.z - q.z;
+    const float d2 = dx * dx + dy * dy + dz * dz;
+    if (j != i && sj != 0 && d2 < best) best = d2;
+  };
+  int bx, by, bz;
+  if (trunc_cell(x.x, x.y, x.z, g, bx, by, bz)) {
+    stencil_rows(bx, by, bz, g, cs, [&](int j0, int j1) {
+      int j = j0;
+      for (; j + 4 <= j1; j += 4) {
+        Packed3 q[4];
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          q[u] = ld3(pos, j + u);
+          v[u] = surf[j + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) test(j + u, q[u], v[u]);
+      }
+      for (; j < j1; ++j) test(j, ld3(pos, j), surf[j]);
+    });
+  }
+  sd[i] = best;
 }
 
 // Start of a marking pass: no claims yet.
@@ -883,8 +929,8 @@ extern "C" int gg_surface(gg_particles *set, const int *cell_start, const gg_par
   prof_begin(GG_STAGE_ADAPTIVE, stream);
   k_radius_surface<<<blocks_for(n), kBlock, 0, stream>>>(n, set->mass, denom, rs);
   GG_LAUNCH_CHECK();
-  k_cover_surface<<<(n + 3) / 4, 64, 0, stream>>>(n, reinterpret_cast<const float *>(set->pos), rs,
-                                                  cell_start, g, set->surface);
+  const float *pos = reinterpret_cast<const float *>(set->pos);
+  k_cover_surface<<<(n + 3) / 4, 64, 0, stream>>>(n, pos, rs, cell_start, g, set->surface);
   GG_LAUNCH_CHECK();
   prof_end(GG_STAGE_ADAPTIVE, stream);
   return GG_OK;
@@ -897,9 +943,13 @@ extern "C" int gg_surface_distance(gg_particles *set, const int *cell_start,
   const int n = set->n;
   if (n == 0) return GG_OK;
   prof_begin(GG_STAGE_ADAPTIVE, stream);
-  k_surface_distance<<<(n + 3) / 4, 64, 0, stream>>>(
-      n, reinterpret_cast<const float *>(set->pos), set->surface, cell_start,
-      dev_grid(ws->grid), set->surface_distance);
+  const float *pos = reinterpret_cast<const float *>(set->pos);
+  if (n <= kGroupDistanceMax)
+    k_surface_distance<<<(n + 3) / 4, 64, 0, stream>>>(
+        n, pos, set->surface, cell_start, dev_grid(ws->grid), set->surface_distance);
+  else
+    k_surface_distance_lane<<<blocks_for(n), kBlock, 0, stream>>>(
+        n, pos, set->surface, cell_start, dev_grid(ws->grid), set->surface_distance);
   GG_LAUNCH_CHECK();
   prof_end(GG_STAGE_ADAPTIVE, stream);
   return GG_OK;

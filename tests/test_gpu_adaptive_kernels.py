@@ -93,6 +93,29 @@ def test_stencil_passes_equal_oracle(gpu, n, crowd):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("n", [262144, 262145, 270001])
+def test_surface_distance_on_both_sides_of_its_rule(gpu, n):
+    # (16 lanes a particle up to 262,144, one above)
+    from granular_gpu_amd import _lib
+    from granular_gpu_amd.device import _ptr, _stream
+    rng = np.random.default_rng(n)
+    cells = (30, 31, 33)
+    L = float(scenes.CELL_LENGTH)
+    pos = rng.random((n, 3)) * (np.array(cells) * L)
+    pos[:2000] = 0.5 + 0.05 * rng.random((2000, 3))
+    pos[2000:2100] += 40.0  # outside the grid
+    pos[2100] = np.nan
+    s = _scene(pos, np.ones(n), cells)
+    sim, pos, vel, mass, cs = _sorted_sim(s)
+    surf = (rng.random(n) < 0.1).astype(np.int32)
+    sim.surface[:n] = torch.from_numpy(surf).cuda()
+    _lib.check("gg_surface_distance", sim.lib.gg_surface_distance(
+        C.byref(sim.set), _ptr(sim.cs), C.byref(sim.ws), _stream()))
+    sd = np.zeros(n, np.float32)
+    po.load().oracle_surface_distance(n, pos.reshape(-1), surf, cs, po.params_from(s, 3, 5), sd)
+    assert np.array_equal(sim.sd[:n].cpu().numpy(), sd)
+
+
 def test_positions_and_masses_that_are_not_finite(gpu):
     from granular_gpu_amd import _lib
     from granular_gpu_amd.device import _ptr, _stream
