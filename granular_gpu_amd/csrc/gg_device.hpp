@@ -129,36 +129,32 @@ __device__ __forceinline__ void stencil_rows(int bx, int by, int bz, const DevGr
   }
 }
 
-// The index ranges [a, b) over two cell tables of the nine rows of a stencil,
-// in scan order, each loaded one row ahead of its use: f(a0, b0, a1, b1) is
-// called per row (empty ranges included), so a scan waits for one round of
-// table loads, not for one per row.
+// The index ranges [a, b) of the nine rows of a stencil, in scan order, each
+// loaded one row ahead of its use: f(a, b) is called per row (empty ranges
+// included), so a scan waits for one round of table loads, not for one per
+// row.
 template <class F>
 __device__ __forceinline__ void stencil_rows_ahead(bool ok, int bx, int by, int bz,
-                                                   const DevGrid &g, const int *__restrict__ t0,
-                                                   const int *__restrict__ t1, F &&f) {
+                                                   const DevGrid &g, const int *__restrict__ cs,
+                                                   F &&f) {
   const int z0 = bz - 1 > 0 ? bz - 1 : 0;
   const int z1 = bz + 1 < g.cz - 1 ? bz + 1 : g.cz - 1;
-  int n0 = 0, m0 = 0, n1 = 0, m1 = 0;
+  int na = 0, nb = 0;
   auto load = [&](int r) {
-    n0 = m0 = n1 = m1 = 0;
+    na = nb = 0;
     const int x = bx + r / 3 - 1, y = by + r % 3 - 1;
     if (ok && z0 <= z1 && x >= 0 && x < g.cx && y >= 0 && y < g.cy) {
       const int c = (x * g.cy + y) * g.cz;
-      n0 = t0[c + z0];
-      m0 = t0[c + z1 + 1];
-      if (t1) {
-        n1 = t1[c + z0];
-        m1 = t1[c + z1 + 1];
-      }
+      na = cs[c + z0];
+      nb = cs[c + z1 + 1];
     }
   };
   load(0);
 #pragma unroll 1
   for (int r = 0; r < 9; ++r) {
-    const int a0 = n0, b0 = m0, a1 = n1, b1 = m1;
+    const int a = na, b = nb;
     if (r < 8) load(r + 1);
-    f(a0, b0, a1, b1);
+    f(a, b);
   }
 }
 

@@ -428,7 +428,7 @@ __global__ void __launch_bounds__(256)
   // 64k coarse particles took 126 us; now 94)
   int bx = 0, by = 0, bz = 0;
   const bool ok = floor_cell(qx, qy, qz, fg, bx, by, bz);
-  stencil_rows_ahead(ok, bx, by, bz, fg, fcs, nullptr, [&](int j0, int j1, int, int) {
+  stencil_rows_ahead(ok, bx, by, bz, fg, fcs, [&](int j0, int j1) {
     for (int j = j0; j < j1; j += 8) {
       Packed3 f[8];
 #pragma unroll

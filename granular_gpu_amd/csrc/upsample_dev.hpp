@@ -13,79 +13,19 @@ struct UpConst {
   float dt, gdx, gdy, gdz, r9, brad, rep, minw, neard, groundy, groundd, vmax, floory, floorf;
 };
 
-// EXACT: the full square root; else the short one (gg_device.hpp), raising
-// odd for a squared distance outside its domain.
-template <bool EXACT>
-__device__ __forceinline__ float distance(float d2, bool &odd) {
-  if (EXACT) return sqrtf(d2);
-  odd |= __float_as_uint(d2) - kSqrtFastMinBits > 0x7f7fffffu - kSqrtFastMinBits;
-  return sqrt_core(d2);
-}
-
-struct UpSums {
-  float wx, wy, wz, gw, maxw, rx, ry, rz;
-  bool near;
-};
-
-// The sums over the coarse particles and the walls around (px, py, pz), each
-// in scan order.  A row (three cells, a handful of coarse particles) is
-// loaded four particles at a time: one round of loads per row.
-template <bool EXACT>
-__device__ __forceinline__ bool upsample_sums(float px, float py, float pz,
-                                              const float *__restrict__ cpos,
-                                              const float *__restrict__ cvel,
-                                              const int *__restrict__ cs,
-                                              const float *__restrict__ bpos,
-                                              const int *__restrict__ bcs, const DevGrid &g,
-                                              const UpConst &u, UpSums &s) {
-  s = UpSums{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, false};
-  bool odd = false;
-  int bx = 0, by = 0, bz = 0;
-  const bool ok = floor_cell(px, py, pz, g, bx, by, bz);
-  stencil_rows_ahead(ok, bx, by, bz, g, cs, bcs, [&](int j0, int j1, int k0, int k1) {
-    for (int j = j0; j < j1; j += 4) {
-      Packed3 a[4], v[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int jt = j + t < j1 ? j + t : j;
-        a[t] = ld3(cpos, jt);
-        v[t] = ld3(cvel, jt);
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if (j + t >= j1) continue;
-        const float dx = px - a[t].x, dy = py - a[t].y, dz = pz - a[t].z;
-        const float dis = distance<EXACT>(dx * dx + dy * dy + dz * dz, odd);
-        const float t1 = 1.0f - dis * dis * u.r9;
-        const float w = fmaxf(0.0f, t1 * t1 * t1);
-        s.gw = s.gw + w;
-        s.wx = s.wx + w * v[t].x;
-        s.wy = s.wy + w * v[t].y;
-        s.wz = s.wz + w * v[t].z;
-        s.maxw = fmaxf(s.maxw, w);
-      }
-    }
-    for (int k = k0; k < k1; k += 4) {
-      Packed3 q[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) q[t] = ld3(bpos, k + t < k1 ? k + t : k);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if (k + t >= k1) continue;
-        const float tx = px - q[t].x, ty = py - q[t].y, tz = pz - q[t].z;
-        const float dis = distance<EXACT>(tx * tx + ty * ty + tz * tz, odd);
-        if (dis < u.brad) {
-          s.near = true;
-          const float den = dis + 1e-6f;
-          const float force = (u.rep * (u.brad - dis)) / u.brad;
-          s.rx = s.rx + (tx / den) * force;
-          s.ry = s.ry + (ty / den) * force;
-          s.rz = s.rz + (tz / den) * force;
-        }
-      }
-    }
-  });
-  return odd;
+__device__ __forceinline__ void coarse_term(float px, float py, float pz, float cx, float cy,
+                                            float cz, float vx, float vy, float vz, float r9,
+                                            float &gw, float &wx, float &wy, float &wz,
+                                            float &maxw) {
+  const float dx = px - cx, dy = py - cy, dz = pz - cz;
+  const float dis = sqrtf(dx * dx + dy * dy + dz * dz);
+  const float t1 = 1.0f - dis * dis * r9;
+  const float w = fmaxf(0.0f, t1 * t1 * t1);
+  gw = gw + w;
+  wx = wx + w * vx;
+  wy = wy + w * vy;
+  wz = wz + w * vz;
+  maxw = fmaxf(maxw, w);
 }
 
 // Position (px,py,pz) and velocity (vix,viy,viz) in; new position and
@@ -96,13 +36,49 @@ __device__ __forceinline__ void upsample_one(
     const float *__restrict__ bpos, const int *__restrict__ bcs, const DevGrid &g,
     const UpConst &u, float &nx_out, float &ny_out, float &nz_out, float &vx_out, float &vy_out,
     float &vz_out) {
-  UpSums s;
-  // (coincident positions, or non-finite ones: again with the full root)
-  if (upsample_sums<false>(px, py, pz, cpos, cvel, cs, bpos, bcs, g, u, s))
-    upsample_sums<true>(px, py, pz, cpos, cvel, cs, bpos, bcs, g, u, s);
-  float wx = s.wx, wy = s.wy, wz = s.wz;
-  const float gw = s.gw, maxw = s.maxw, rx = s.rx, ry = s.ry, rz = s.rz;
-  const bool near = s.near;
+  float wx = 0.0f, wy = 0.0f, wz = 0.0f, gw = 0.0f, maxw = 0.0f;
+  float rx = 0.0f, ry = 0.0f, rz = 0.0f;
+  bool near = false;
+  int bx, by, bz;
+  if (floor_cell(px, py, pz, g, bx, by, bz)) {
+    stencil_rows(bx, by, bz, g, cs, [&](int j0, int j1) {
+      int j = j0;
+      for (; j + 2 <= j1; j += 2) {
+        const Packed3 a = ld3(cpos, j), b = ld3(cpos, j + 1);
+        const Packed3 v = ld3(cvel, j), w = ld3(cvel, j + 1);
+        coarse_term(px, py, pz, a.x, a.y, a.z, v.x, v.y, v.z, u.r9, gw, wx, wy, wz, maxw);
+        coarse_term(px, py, pz, b.x, b.y, b.z, w.x, w.y, w.z, u.r9, gw, wx, wy, wz, maxw);
+      }
+      for (; j < j1; ++j) {
+        const Packed3 a = ld3(cpos, j), v = ld3(cvel, j);
+        coarse_term(px, py, pz, a.x, a.y, a.z, v.x, v.y, v.z, u.r9, gw, wx, wy, wz, maxw);
+      }
+    });
+    auto wall = [&](const Packed3 &q) {
+      const float tx = px - q.x, ty = py - q.y, tz = pz - q.z;
+      const float dis = sqrtf(tx * tx + ty * ty + tz * tz);
+      if (dis < u.brad) {
+        near = true;
+        const float den = dis + 1e-6f;
+        const float force = (u.rep * (u.brad - dis)) / u.brad;
+        rx = rx + (tx / den) * force;
+        ry = ry + (ty / den) * force;
+        rz = rz + (tz / den) * force;
+      }
+    };
+    stencil_rows(bx, by, bz, g, bcs, [&](int k0, int k1) {
+      int k = k0;
+      for (; k + 4 <= k1; k += 4) {
+        const Packed3 q0 = ld3(bpos, k), q1 = ld3(bpos, k + 1), q2 = ld3(bpos, k + 2),
+                      q3 = ld3(bpos, k + 3);
+        wall(q0);
+        wall(q1);
+        wall(q2);
+        wall(q3);
+      }
+      for (; k < k1; ++k) wall(ld3(bpos, k));
+    });
+  }
   float vx, vy, vz;
   if (gw > u.minw) {
     wx = wx / gw;
