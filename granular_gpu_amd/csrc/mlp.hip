@@ -1422,7 +1422,7 @@ struct SideStream {
   hipStream_t st = nullptr;
   hipEvent_t fork = nullptr, join = nullptr, flags = nullptr;
 };
-constexpr int kFlagsFirst = 262144;
+constexpr int kFlagsFirst = 98304;
 static int side_stream(SideStream *&out) {
   static SideStream per_dev[64];
   int dev = 0;
@@ -1487,9 +1487,12 @@ extern "C" int gg_upsample_mlp(const gg_particles *coarse, const int *cs,
   // stream (disjoint outputs); the network waits for the flags only.  Fused
   // into the features pass instead, the fallback would start only after it.
   // Up to kFlagsFirst particles the flags come first on the caller's stream
-  // instead: a wait between streams costs more than the overlap gives (27k
-  // 68.6 -> 62.0 us a call, 92k 82.1 -> 79.4, 216k 96.3 -> 94.2; at 332k
-  // side by side is ahead, 116.8 against 121.9, at 512k 150.8 against 159.7).
+  // instead: a wait between streams costs more than the overlap gives.  With
+  // nothing flagged that holds to some 200k (27k 68.6 -> 62.0 us a call, 92k
+  // 82.1 -> 79.4, 216k 96.3 -> 94.2), but in a settled pile, where up to a
+  // third is flagged and the fallback is as long as the rest, starting it
+  // before the features costs: 27k 77.8 -> 72.9, 91k 107.9 -> 106.0, 125k
+  // 117.5 -> 119.1, 216k 157 -> 172, 250k 171 -> 193.
   SideStream *side = nullptr;
   GG_TRY(side_stream(side));
   std::lock_guard<std::mutex> lock(side->mu);
