@@ -992,7 +992,9 @@ static int merge_mark_rules(gg_particles *set, gg_adaptive *ad, const int *cell_
                                                max_mass, R, rs, cand, dens, state, und[0]);
   GG_LAUNCH_CHECK();
   // about kMergeRounds rounds bring a hundred thousand claims down to what
-  // the finisher holds on chip; one more for every quarter more of them
+  // the finisher holds on chip; one more for every quarter more of them.
+  // Marking jittered lattices with 7, this many and 14: 32,768 particles 0.28,
+  // 0.20 and 0.17 ms, 140,608 1.01, 0.65 and 0.38, 1M 3.7, 1.84 and 1.32.
   int rounds = kMergeRounds;
   for (long long k = kMergeSet; k < n && rounds < 2 * kMergeRounds; k += k / 4) ++rounds;
   for (int r = 0; r < rounds; ++r) {

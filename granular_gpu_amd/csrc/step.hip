@@ -16,15 +16,19 @@
 // D = x* - x stays small, so differences and the final x = base + D are
 // rounded once.
 //
-// Neighbour candidate lists: built once per step with a skin; a sweep uses
-// particle i's list only when (a) the stencil base of x*_i is the one the
-// list was built for and (b) i's accumulated displacement plus the largest
-// displacement of any particle is below 0.9*skin, which guarantees every
-// pair outside the list is still out of contact.  Otherwise the particle
-// scans the full 27-cell stencil, in its own lane or, when few lanes of its
-// wave need to, queued and scanned by a whole wave in a second pass.  All paths
-// visit contacts in the same order, so the result is identical to always
-// scanning the stencil.
+// Neighbour candidate lists: built once per step with a skin (and, with the
+// refresh, again within it); a sweep uses particle i's list only when (a) the
+// stencil base of x*_i is the one the list was built for, or one cell over
+// where no pair in reach can have entered or left, and (b) i's displacement
+// plus the largest of its stencil is below 0.9 skin, which guarantees that
+// every pair outside the list is still out of contact.  The largest is 0.45
+// skin unless a particle beyond that has marked the cells around it with its
+// own.  The near list, the entries within 0.7 skin, takes the list's place
+// while the two displacements add up to less than 0.6 skin.  Otherwise the
+// particle scans the full 27-cell stencil, in its own lane or, when few lanes
+// of its wave need to, queued in the block's LDS and scanned by a whole wave.
+// All paths visit contacts in the same order, so the result is identical to
+// always scanning the stencil.
 #include <hip/hip_runtime.h>
 
 #include "gg_device.hpp"
@@ -218,7 +222,7 @@ __device__ __forceinline__ int boundary_list(const ListArgs &a, const DevGrid &g
 // order.  A particle whose own limit does not fit the quantised form looks at
 // every candidate; one whose radius does not (4 cells) marks the cells around
 // it, so that nobody there uses a list that may lack it.  1M particles: 178
-// -> 134 us.
+// -> 135 us.
 constexpr int kListChunk = 24;  // candidates per mask (a row of three cells holds about as many)
 template <int BS, bool SCENES>
 __global__ void __launch_bounds__(BS) k_nlist(ListArgs a) {
@@ -803,13 +807,12 @@ __device__ __forceinline__ void scan_by_wave(const SweepArgs &a, int iq) {
 // gathers (the first eight beside the particle's own state), and the contact
 // arithmetic takes the short branch-free sequences of fast_terms.  5 waves
 // per SIMD: the entries' registers are worth more than a sixth wave.  1M
-// particles, friction: 46.8 -> 34.4 us; without: 41.0 -> 29.6 us; 1.7k
-// particles, without: 8.7 -> 5.9 us.
-// One sweep.  Particles whose candidate list is provably exact for this
-// sweep use it; the others scan the full stencil, either in their own lane
-// or (when few lanes of the wave need it) queued for k_sweep_queue, which
-// scans each with a whole wave.  All paths visit contacts in
-// the same order, so the result does not depend on which path ran.
+// particles, friction: 46.8 -> 34.8 us; without: 41.0 -> 28.9 us; 1.7k
+// particles, without: 8.7 -> 5.9 us; sets that mostly scan stencils (the
+// excavator's 1.9M) 1475 -> 1487 us.  Particles whose lists lapsed scan the
+// stencil in their own lane or, when few lanes of the wave need it, queued in
+// the block's LDS for whole waves after the list work (sweep-wide, for
+// k_sweep_queue, only when asked for).
 template <bool FRIC, bool LAST_STAB, int BS, bool SCENES>
 __global__ void __launch_bounds__(BS, 5) k_sweep(SweepArgs a) {
   __shared__ int lqueue[BS];
@@ -977,7 +980,10 @@ __device__ __forceinline__ void add_quad(float3 &acc, const float3 &c, const flo
 // across the four lanes in list order.  A third more instructions per
 // particle.  Particles whose lists lapsed are scanned by the wave.
 // Measured (k_sweep, this; a launch is 4 of it): 1.7k particles 5.9, 5.0 us;
-// 33k with friction 7.7, 7.0; 111k 8.0, 9.8.
+// 33k with friction 7.7, 7.0; 111k 8.0, 9.8.  Whole steps of a settling block,
+// captured, without and with friction: 46,656 particles 344, 327 and 289, 239
+// us; 54,872 401, 355 and 310, 259; 64,000 395, 407 and 338, 288; 85,184 396,
+// 560 and 366, 370: they cross at about 60k and 85k.
 constexpr int kQuadSweepMax = 49152;
 template <bool FRIC, bool LAST_STAB, bool SCENES>
 __global__ void __launch_bounds__(64) k_sweep_quad(SweepArgs a) {

@@ -437,7 +437,10 @@ int gg_mlp_teacher(const gg_particles *coarse, const int *cell_start,
 int gg_mlp_fine_targets(const gg_particles *coarse, const gg_particles *fine,
                         const int *fine_cell_start, gg_grid fine_grid, const gg_mlp_config *c,
                         float *y, float *d2, int *match, hipStream_t stream);
-/* Training path (MFMA GEMMs, scratch of gg_mlp_train_scratch_bytes(B)). */
+/* Training path: the whole network in one kernel each way, scratch of
+ * gg_mlp_train_scratch_bytes(B) (at least 5376 bytes per sample).  A gradient
+ * is a sum of as many partial gradients as the scratch holds, so its last bits
+ * are the same from call to call for the same batch and scratch size only. */
 size_t gg_mlp_train_scratch_bytes(int batch);
 int gg_mlp_forward(const gg_mlp_weights *w, const uint16_t *x, int batch, float *y,
                    void *scratch, size_t scratch_bytes, hipStream_t stream);
